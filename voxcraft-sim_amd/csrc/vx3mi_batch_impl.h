@@ -406,15 +406,10 @@ template <typename T> __device__ __forceinline__ V3<T> col_diff(const T4<T> &pv,
     return V3<T>{(T)(-o.x) * L + (pv.x - pw.x), (T)(-o.y) * L + (pv.y - pw.y), (T)(-o.z) * L + (pv.z - pw.z)};
 }
 
-// rebuild pass 1 (robots whose lists are stale): the cell of each surface voxel,
-// its rank within its bucket, its position field at the listing
-template <typename T> __device__ __forceinline__ void col_count(const Dev<T> &a, int s, int parity) {
-    const int v = a.surf[s];
-    const int r = a.vrob[v];
-    const RobotTime *rt = a.rt + r;
-    if (!rt->stale[parity] || rt->diverged) return;
-    const RobotParams &rp = a.rp[r];
-    const T4<T> q0 = a.pq0[v];
+// surface voxel s (voxel v) at position field q0 counted into its bucket: its
+// cell, its rank within the bucket, its position field at the listing
+template <typename T>
+__device__ __forceinline__ void col_cell(const Dev<T> &a, const RobotParams &rp, int s, int v, const T4<T> &q0) {
     const V3<double> p = position_d<T>(a.lat[v], a.vmats[a.vmat[v]].nomSize, V3<T>{q0.x, q0.y, q0.z});
     const double h = rp.listR;
     const int cx = (int)floor(p.x / h), cy = (int)floor(p.y / h), cz = (int)floor(p.z / h);
@@ -422,6 +417,15 @@ template <typename T> __device__ __forceinline__ void col_count(const Dev<T> &a,
     a.scell[s] = int4{cx, cy, cz, key};
     a.srank[s] = atomicAdd(&a.ccnt[rp.toff + key], 1);
     a.bpos[v] = q0;
+}
+
+// rebuild pass 1 (robots whose lists are stale)
+template <typename T> __device__ __forceinline__ void col_count(const Dev<T> &a, int s, int parity) {
+    const int v = a.surf[s];
+    const int r = a.vrob[v];
+    const RobotTime *rt = a.rt + r;
+    if (!rt->stale[parity] || rt->diverged) return;
+    col_cell(a, a.rp[r], s, v, a.pq0[v]);
 }
 
 // rebuild pass 2, one workgroup of blockDim threads (a multiple of 64, at most
@@ -493,18 +497,22 @@ template <bool WIDE, typename T> __device__ __forceinline__ void col_scan(const 
     }
 }
 
-// rebuild pass 3: surface indices (robot-relative) in bucket order
-template <typename T> __device__ __forceinline__ void col_scatter(const Dev<T> &a, int s, int parity) {
-    const int v = a.surf[s];
-    const int r = a.vrob[v];
-    const RobotTime *rt = a.rt + r;
-    if (!rt->stale[parity] || rt->diverged) return;
-    const RobotParams &rp = a.rp[r];
+// surface voxel s (voxel v): its record at its place in bucket order
+template <typename T> __device__ __forceinline__ void col_record(const Dev<T> &a, const RobotParams &rp, int s, int v) {
     const int4 c = a.scell[s];
     const int k = rp.soff + a.cstart[rp.toff + c.w] + a.srank[s];
     const T4<T> q = a.bpos[v];
     a.grec[k] = int4{c.x, c.y, c.z, v};
     a.gpos[k] = T4<T>{q.x, q.y, q.z, lat_word<T>(a.lat[v])};
+}
+
+// rebuild pass 3: the records of the robots whose lists are stale
+template <typename T> __device__ __forceinline__ void col_scatter(const Dev<T> &a, int s, int parity) {
+    const int v = a.surf[s];
+    const int r = a.vrob[v];
+    const RobotTime *rt = a.rt + r;
+    if (!rt->stale[parity] || rt->diverged) return;
+    col_record(a, a.rp[r], s, v);
 }
 
 // calls f(w, pw) for every surface voxel w of the robot in the 27 grid cells
