@@ -1339,6 +1339,7 @@ template <typename T> struct Batch : BatchBase {
     struct TilePlan {
         bool ok = false;
         int ntiles = 0;
+        int maxLinks = 0;         // of the fullest tile
         int4 *d_tiles = nullptr;  // robot begin, robot count, voxels, links
         int *d_tileRobots = nullptr;
     } plans[2];                   // large and small tile configuration
@@ -1827,7 +1828,7 @@ template <typename T> struct Batch : BatchBase {
         using C = typename TileSel<T, SMALL, COL>::C;
         TilePlan &P = plans[SMALL];
         P.ok = false;
-        if (anyForceField || anyCilia || plainFlatOnly() || R < 2) return VX3MI_OK;
+        if (anyForceField || anyCilia || plainFlatOnly() || V == 0) return VX3MI_OK;
         if (anyCollisions && SMALL) return VX3MI_OK;  // collision tiles: the large configuration
         long totL = 0, totV = 0;
         for (const RobotParams &p : hrp) {
@@ -1841,31 +1842,45 @@ template <typename T> struct Batch : BatchBase {
             if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) cus = prop.multiProcessorCount;
         }
         const long slots = (long)cus * (SMALL ? 2 : 1);
-        long want = std::max<long>({slots, (totL + C::LMAX - 1) / C::LMAX, (totV + C::VMAX - 1) / C::VMAX});
-        want = std::min<long>(want, R);
+        // A launch lasts as many rounds as its fullest workgroup slot runs tiles,
+        // so the tiles are one round of the device, or else the fewest whole
+        // rounds that hold the batch.  Robots go, longest first, to the least
+        // loaded tile with room; where that leaves one over (a batch that nearly
+        // fills its tiles), to the fullest tile with room, which leaves the small
+        // robots for the gaps.
+        struct Bin { long l = 0, v = 0; std::vector<int> robots; };
+        std::vector<Bin> bins;
         std::vector<int> order(R);
         for (int r = 0; r < R; r++) order[r] = r;
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hrp[x].lcount > hrp[y].lcount; });
-        struct Bin { long l = 0, v = 0; std::vector<int> robots; };
-        std::vector<Bin> bins((size_t)want);
-        for (int r : order) {
-            const RobotParams &p = hrp[r];
-            int best = -1;
-            for (int b = 0; b < (int)bins.size(); b++) {
-                const Bin &x = bins[b];
-                if (x.l + p.lcount > C::LMAX || x.v + p.vcount > C::VMAX || (int)x.robots.size() >= C::RMAX) continue;
-                if (best < 0 || x.l + x.v < bins[best].l + bins[best].v) best = b;
+        auto pack = [&](long n, bool full) {
+            bins.assign((size_t)n, Bin());
+            for (int r : order) {
+                const RobotParams &p = hrp[r];
+                int best = -1;
+                for (int b = 0; b < (int)bins.size(); b++) {
+                    const Bin &x = bins[b];
+                    if (x.l + p.lcount > C::LMAX || x.v + p.vcount > C::VMAX || (int)x.robots.size() >= C::RMAX) continue;
+                    if (best < 0 || (full ? x.l + x.v > bins[best].l + bins[best].v : x.l + x.v < bins[best].l + bins[best].v)) best = b;
+                }
+                if (best < 0) return false;
+                bins[best].l += p.lcount;
+                bins[best].v += p.vcount;
+                bins[best].robots.push_back(r);
             }
-            if (best < 0) { bins.emplace_back(); best = (int)bins.size() - 1; }
-            bins[best].l += p.lcount;
-            bins[best].v += p.vcount;
-            bins[best].robots.push_back(r);
+            return true;
+        };
+        const long least = std::max((totL + C::LMAX - 1) / C::LMAX, (totV + C::VMAX - 1) / C::VMAX);
+        for (long rounds = std::max<long>(1, (least + slots - 1) / slots);; rounds++) {
+            const long n = std::min<long>(rounds * slots, R);
+            if (pack(n, false) || pack(n, true)) break;  // (a tile for each robot always holds them)
         }
         std::vector<int4> tiles;
         std::vector<int> trobots;
         for (Bin &b : bins) {
             if (b.robots.empty()) continue;
             std::sort(b.robots.begin(), b.robots.end());
+            P.maxLinks = std::max(P.maxLinks, (int)b.l);
             tiles.push_back(int4{(int)trobots.size(), (int)b.robots.size(), (int)b.v, (int)b.l});
             for (int r : b.robots) trobots.push_back(r);
         }
@@ -1886,8 +1901,22 @@ template <typename T> struct Batch : BatchBase {
         if (rc || (rc = plan_tiles_cfg<1, 0>())) return rc;
         tileOK = plans[0].ok || plans[1].ok;
         tileSel = plans[0].ok ? 0 : 1;
-        autoMode = tileOK ? VX3MI_MODE_TILED
-                          : ((R > 1 && V / R <= 4096 && !plainFlatOnly()) ? VX3MI_MODE_PERSISTENT : VX3MI_MODE_FLAT);
+        // The mode of a batch that is not tuned.  A tile's step takes a time that
+        // grows with its links, a flat step one that grows with the whole batch
+        // but starts higher (its launches): microseconds per step, fitted to
+        // batches of 1..400 robots of 3..16 voxels per axis (one robot of 784
+        // voxels, 1,655 links with collisions in FP32: 16.4 tiled, 12.9 flat;
+        // 270 voxels, 550 links: 7.7 and 12.7).  Batches with a robot no tile
+        // holds go flat too: the per-robot kernel is as slow as its largest robot
+        // (200 robots of up to 1,533 links in FP64: 76-119 with 512-256 threads,
+        // flat 69).
+        constexpr bool f32 = std::is_same<T, float>::value;
+        const bool col = anyCollisions;
+        const double tile0 = f32 ? (col ? 4.5 : 3.0) : (col ? 6.4 : 5.5);
+        const double tileLink = f32 ? (col ? 6.6e-3 : 3.3e-3) : (col ? 15.5e-3 : 10.8e-3);
+        const double flat0 = f32 ? (col ? 12.8 : 8.5) : (col ? 16.3 : 14.2), flatVoxel = col ? 1.1e-3 : 8e-5;
+        const bool tiled = tileOK && tile0 + tileLink * plans[tileSel].maxLinks <= flat0 + flatVoxel * V;
+        autoMode = tiled ? VX3MI_MODE_TILED : VX3MI_MODE_FLAT;
         return VX3MI_OK;
     }
 
