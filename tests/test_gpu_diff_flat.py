@@ -1,0 +1,46 @@
+"""Differentiable steps as launches over the whole batch: a small robot gives the
+same bits in a batch with a large one (flat steps) as alone (one workgroup per
+robot), forward state and gradients, with the whole tape kept and with
+checkpoints, at step counts on both sides of a checkpoint."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path[:0] = [os.path.join(ROOT, "voxcraft-sim_amd")]
+
+import vx3mi  # noqa: E402
+from vx3mi import configs  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (4, 3, 3), (5, 5, 3)])
+@pytest.mark.parametrize("every,steps", [(0, 1), (0, 41), (13, 39), (13, 40), (40, 40)])
+def test_flat_steps_equal_a_workgroup_per_robot(precision, dims, every, steps):
+    small, large = configs.config3(seed=2, dims=dims), configs.config3(seed=3, dims=(11, 9, 9))
+    ms, ml = vx3mi.Model.from_problem(small), vx3mi.Model.from_problem(large)
+    assert ml.nl > 2 * 650 > 4 * ms.nl  # on either side of where the two ways cost the same
+    out = []
+    g = np.random.default_rng(1).normal(size=(ms.nv, 10))
+    for models in ([ms], [ms, ml], [ml, ms]):
+        d = vx3mi.Diff(models, precision, checkpoint_every=every)
+        at = sum(m.nv for m in models[:models.index(ms)])
+        d.forward(steps)
+        s = d.state(models.index(ms))
+        bars = []
+        for a, b in ((0, 3), (3, 7), (7, 10)):
+            full = np.zeros((d.nv, b - a))
+            full[at:at + ms.nv] = g[:, a:b]
+            bars.append(full)
+        gp, ge = d.backward(grad_pos=bars[0], grad_quat=bars[1], grad_linmom=bars[2])
+        out.append((s, gp[at:at + ms.nv], ge[at:at + ms.nv]))
+        d.close()
+    for s, gp, ge in out[1:]:
+        for k in s:
+            assert np.array_equal(s[k], out[0][0][k]), k
+        np.testing.assert_array_equal(gp, out[0][1])
+        np.testing.assert_array_equal(ge, out[0][2])

@@ -68,6 +68,26 @@ __global__ __launch_bounds__(NT) void k_diff_forward(DD<T> d, const RobotParams 
     }
 }
 
+// the same forward step n over every robot at once, one item per thread, two
+// launches in stream order instead of the workgroup barriers: the link phase ...
+// (ck, tape: where the state entering the step goes, or null)
+template <typename T>
+__global__ __launch_bounds__(256) void k_diff_fwd_links(DD<T> d, int n, T4<T> *ckL, T4<T> *tapeL) {
+    const int l = blockIdx.x * blockDim.x + threadIdx.x;
+    if (l >= d.L) return;
+    if (ckL) diff_save_link(d, l, ckL + (size_t)l * 3);
+    if (tapeL) diff_save_link(d, l, tapeL + (size_t)l * 3);
+    diff_link_fwd(d, l, n > 0 ? d.dt : (T)0);
+}
+// ... and the voxel phase
+template <typename T>
+__global__ __launch_bounds__(256) void k_diff_fwd_voxels(DD<T> d, int n, T4<T> *ckV, T4<T> *tapeV) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= d.V) return;
+    if (ckV) diff_save_voxel(d, v, ckV + (size_t)v * 4);
+    diff_voxel_fwd(d, v, d.times[n + 1], tapeV ? tapeV + (size_t)v * 5 : (T4<T> *)nullptr);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_diff_restore(DD<T> d, const T4<T> *ckV, const T4<T> *ckL, int slot) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -149,6 +169,7 @@ template <typename T> struct DiffBatch : DiffBase {
     std::vector<int2v> hends;
     std::vector<int> haxis;
     std::vector<double> hnom;            // link nominal length
+    bool flatSteps = false;              // steps as launches over the whole batch (else one workgroup per robot)
 
     int create(vx3mi_model *const *models, int n, const vx3mi_diff_opts &opts) {
         R = n;
@@ -238,6 +259,23 @@ template <typename T> struct DiffBatch : DiffBase {
         o.varyTemp = m0.varyTemp;
         if (opts.dt > 0) dt = (float)opts.dt;
         else dt = (float)(dtFrac * (maxF2 > 0 ? 1.0f / (6.283185f * std::sqrt(maxF2)) : 1e-10));
+
+        // Whether a step runs as one item per thread over the whole batch, two
+        // launches a phase pair, or as one workgroup per robot: a launch costs more
+        // than a workgroup barrier, a robot's items in turn more than the batch's
+        // side by side.  Microseconds per step, forward and reverse together, as
+        // fitted to 1..1000 robots of 3..16 voxels per axis: FP32, one robot of 141
+        // links 13.5 (robot) and 22 (flat), 675 links 25 and 25, 1,344 links 38 and
+        // 26; 128 robots of up to 3,540 links 126 and 56, of up to 250 links 16 and
+        // 27; 1000 robots of up to 469 links 74 and 59.
+        constexpr bool f32 = std::is_same<T, float>::value;
+        int maxLinks = 0, dev = 0, cus = 256;
+        for (const RobotParams &p : hrp) maxLinks = std::max(maxLinks, p.lcount);
+        hipDeviceProp_t prop;
+        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
+            cus = prop.multiProcessorCount;
+        const double robot = ((f32 ? 12 : 21) + (f32 ? 0.0185 : 0.062) * maxLinks) * ((R + cus - 1) / cus);
+        flatSteps = robot > (f32 ? 24 : 36) + (f32 ? 0.35e-3 : 0.9e-3) * V;
 
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         HIP_TRY(hipStreamCreateWithFlags(&rstream, hipStreamNonBlocking));
@@ -352,6 +390,34 @@ template <typename T> struct DiffBatch : DiffBase {
         return VX3MI_OK;
     }
 
+    // steps [n0, n0 + nsteps) on stream st, a checkpoint every ckEvery steps and /
+    // or a tape whose first slot is step tapeStart
+    // (wide: the workgroup size of the per-robot kernel)
+    void run_forward(hipStream_t st, int n0, int nsteps, bool wide, int ckEvery, T4<T> *cV, T4<T> *cL, T4<T> *tV, T4<T> *tL,
+                     int tapeStart) {
+        if (!flatSteps) {
+            for (int s0 = 0; s0 < nsteps; s0 += chunk) {
+                const int k = std::min(chunk, nsteps - s0);
+                if (wide)
+                    k_diff_forward<T, DiffThreads<T>::FWD><<<R, DiffThreads<T>::FWD, 0, st>>>(d, d_rp, n0 + s0, k, ckEvery, cV, cL,
+                                                                                              tV, tL, tapeStart);
+                else
+                    k_diff_forward<T, DiffThreads<T>::RECOMP><<<R, DiffThreads<T>::RECOMP, 0, st>>>(d, d_rp, n0 + s0, k, ckEvery, cV,
+                                                                                                    cL, tV, tL, tapeStart);
+            }
+            return;
+        }
+        for (int n = n0; n < n0 + nsteps; n++) {
+            const size_t slot = (size_t)(n / ckEvery), ts = (size_t)(n - tapeStart);
+            const bool ck = cV && n % ckEvery == 0;
+            if (L)
+                k_diff_fwd_links<T><<<(L + 255) / 256, 256, 0, st>>>(d, n, ck ? cL + slot * L * 3 : nullptr,
+                                                                     tL ? tL + ts * L * 3 : nullptr);
+            k_diff_fwd_voxels<T><<<(V + 255) / 256, 256, 0, st>>>(d, n, ck ? cV + slot * V * 4 : nullptr,
+                                                                  tV ? tV + ts * V * 5 : nullptr);
+        }
+    }
+
     int forward(int nsteps) override {
         if (nsteps <= 0) { set_error("nsteps must be positive"); return VX3MI_E_ARG; }
         int rc = ensure_buffers(nsteps);
@@ -366,11 +432,7 @@ template <typename T> struct DiffBatch : DiffBase {
         k_diff_init<T><<<std::max(nb, 1), 256, 0, stream>>>(d);
         // the forward keeps checkpoints; with one segment it also writes the tape
         const bool oneSeg = K >= nsteps;
-        for (int s0 = 0; s0 < nsteps; s0 += chunk) {
-            const int k = std::min(chunk, nsteps - s0);
-            k_diff_forward<T, DiffThreads<T>::FWD><<<R, DiffThreads<T>::FWD, 0, stream>>>(
-                d, d_rp, s0, k, K, ckV, ckL, oneSeg ? tapeV : nullptr, oneSeg ? tapeL : nullptr, 0);
-        }
+        run_forward(stream, 0, nsteps, true, K, ckV, ckL, oneSeg ? tapeV : nullptr, oneSeg ? tapeL : nullptr, 0);
         HIP_TRY(hipEventRecord(ev1, stream));
         T4<T> *src[4] = {d.su, d.sq, d.sp, d.sh};
         for (int k = 0; k < 4; k++)
@@ -447,7 +509,7 @@ template <typename T> struct DiffBatch : DiffBase {
         const bool recompute = !(tapeValid && nseg == 1);
         // flat: every robot's reverse step at once over the whole device (a robot
         // larger than the others no longer sets the pace of the sweep)
-        const bool flat = optsIn.reverse_threads < 0;
+        const bool flat = optsIn.reverse_threads < 0 || (optsIn.reverse_threads == 0 && flatSteps);
         const bool wide = flat || (optsIn.reverse_threads == DiffThreads<T>::REV_WIDE &&
                                    DiffThreads<T>::REV_WIDE != DiffThreads<T>::REV);
         hipStream_t rs = rstream;
@@ -457,15 +519,8 @@ template <typename T> struct DiffBatch : DiffBase {
             if (seg + 2 < nseg) HIP_TRY(hipStreamWaitEvent(rs, segEv[4 * (seg + 2) + 3], 0));
             HIP_TRY(hipEventRecord(segEv[4 * seg], rs));
             k_diff_restore<T><<<std::max(nb, 1), 256, 0, rs>>>(d, ckV, ckL, seg);
-            for (int c = 0; c < len; c += chunk) {
-                const int k = std::min(chunk, len - c);
-                if (wide)  // a wide reverse fills the compute units: recompute at full width too
-                    k_diff_forward<T, DiffThreads<T>::FWD><<<R, DiffThreads<T>::FWD, 0, rs>>>(
-                        d, d_rp, s0 + c, k, K, nullptr, nullptr, bufV[seg & 1], bufL[seg & 1], s0);
-                else
-                    k_diff_forward<T, DiffThreads<T>::RECOMP><<<R, DiffThreads<T>::RECOMP, 0, rs>>>(
-                        d, d_rp, s0 + c, k, K, nullptr, nullptr, bufV[seg & 1], bufL[seg & 1], s0);
-            }
+            // (a wide reverse fills the compute units: recompute at full width too)
+            run_forward(rs, s0, len, wide, K, nullptr, nullptr, bufV[seg & 1], bufL[seg & 1], s0);
             HIP_TRY(hipEventRecord(segEv[4 * seg + 1], rs));
             return VX3MI_OK;
         };

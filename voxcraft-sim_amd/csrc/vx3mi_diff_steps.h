@@ -41,6 +41,18 @@ template <typename T> struct DD {
     T *gPhase;
 };
 
+// on the device, an empty asm that takes x as it stands here: the loads of x stay
+// in flight until this point, and no arithmetic on it moves above it (FP32
+// contracts multiplies and adds within a basic block, so where the arithmetic
+// stands decides its rounding)
+template <typename T> VX_HD void hold(T4<T> &x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
+#else
+    (void)x;
+#endif
+}
+
 template <typename T> VX_HD V3<T> xyz(const T4<T> &a) { return V3<T>{a.x, a.y, a.z}; }
 template <typename T> VX_HD Q4<T> wxyz(const T4<T> &a) { return Q4<T>{a.x, a.y, a.z, a.w}; }
 template <typename T> VX_HD T4<T> t4(V3<T> v, T w) { return T4<T>{v.x, v.y, v.z, w}; }
@@ -90,19 +102,20 @@ template <typename T> VX_HD void diff_restore_link(const DD<T> &d, int l, const 
 }
 
 template <typename T> VX_HD void diff_link_fwd(const DD<T> &d, int l, T prevDt) {
+    // (loads before the check that returns early, so that they are in flight with it)
     const DLink<T> &c = d.lc[l];
+    const int2v e = d.lends[l];
+    const T4<T> l0 = d.sl0[l], l1 = d.sl1[l], l2 = d.sl2[l];
+    const T4<T> un = d.su[e.x], up = d.su[e.y], qn = d.sq[e.x], qp = d.sq[e.y];
     if (c.fixedBoth) {
         d.lf0[l] = d.lf1[l] = d.lf2[l] = T4<T>{0, 0, 0, 0};
         return;
     }
-    const int2v e = d.lends[l];
-    const T4<T> un = d.su[e.x], up = d.su[e.y];
     V3<T> P0, A10, A20;
     int flags;
-    unpack_ls(d.sl0[l], d.sl1[l], d.sl2[l], P0, A10, A20, flags);
+    unpack_ls(l0, l1, l2, P0, A10, A20, flags);
     DLinkEval<T> ev;
-    d_link_forward(c, V3<T>{up.x - un.x, up.y - un.y, up.z - un.z}, wxyz(d.sq[e.x]), wxyz(d.sq[e.y]), un.w, up.w, P0, A10,
-                   A20, flags, prevDt, ev);
+    d_link_forward(c, V3<T>{up.x - un.x, up.y - un.y, up.z - un.z}, wxyz(qn), wxyz(qp), un.w, up.w, P0, A10, A20, flags, prevDt, ev);
     d.sl0[l] = t4(ev.P, ev.A1v.x);
     d.sl1[l] = T4<T>{ev.A1v.y, ev.A1v.z, ev.A2v.x, ev.A2v.y};
     d.sl2[l] = T4<T>{ev.A2v.z, (T)ev.flagsOut, 0, 0};
@@ -114,17 +127,25 @@ template <typename T> VX_HD void diff_link_fwd(const DD<T> &d, int l, T prevDt) 
 template <typename T> VX_HD void gather_forces(const DD<T> &d, int v, V3<T> &F, V3<T> &M) {
     F = V3<T>{0, 0, 0};
     M = V3<T>{0, 0, 0};
+    int vl[6];
+    T4<T> a[6], b[6];  // every link's words in flight at once, summed in direction order
+#pragma unroll
+    for (int k = 0; k < 6; k++) vl[k] = d.vlinks[6 * v + k];
+#pragma unroll
     for (int k = 0; k < 6; k++) {
-        const int l = d.vlinks[6 * v + k];
-        if (l < 0) continue;
-        if (k & 1) {  // this voxel is the link's pVPos end
-            const T4<T> f1 = d.lf1[l], f2 = d.lf2[l];
-            F = F + V3<T>{f1.z, f1.w, f2.x};
-            M = M + V3<T>{f2.y, f2.z, f2.w};
+        if (vl[k] < 0) continue;
+        a[k] = (k & 1) ? d.lf1[vl[k]] : d.lf0[vl[k]];  // odd: this voxel is the link's pVPos end
+        b[k] = (k & 1) ? d.lf2[vl[k]] : d.lf1[vl[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        if (vl[k] < 0) continue;
+        if (k & 1) {
+            F = F + V3<T>{a[k].z, a[k].w, b[k].x};
+            M = M + V3<T>{b[k].y, b[k].z, b[k].w};
         } else {
-            const T4<T> f0 = d.lf0[l], f1 = d.lf1[l];
-            F = F + V3<T>{f0.x, f0.y, f0.z};
-            M = M + V3<T>{f0.w, f1.x, f1.y};
+            F = F + V3<T>{a[k].x, a[k].y, a[k].z};
+            M = M + V3<T>{a[k].w, b[k].x, b[k].y};
         }
     }
 }
@@ -132,17 +153,21 @@ template <typename T> VX_HD void gather_forces(const DD<T> &d, int v, V3<T> &F, 
 // voxel phase of step n; tape (5 T4 of this voxel's slot, or null) receives
 // the state entering the step and the force sums
 template <typename T> VX_HD void diff_voxel_fwd(const DD<T> &d, int v, double tNext, T4<T> *tape) {
+    T4<T> u = d.su[v], q = d.sq[v], p = d.sp[v], h = d.sh[v];
     V3<T> F, M;
     gather_forces(d, v, F, M);
-    const T4<T> u = d.su[v];
+    hold(u);
+    hold(q);
+    hold(p);
+    hold(h);
     DVoxState<T> s, out;
     s.u = xyz(u);
-    s.q = wxyz(d.sq[v]);
-    s.p = xyz(d.sp[v]);
-    s.h = xyz(d.sh[v]);
+    s.q = wxyz(q);
+    s.p = xyz(p);
+    s.h = xyz(h);
     if (tape) {
         tape[0] = u;
-        tape[1] = d.sq[v];
+        tape[1] = q;
         tape[2] = t4(s.p, F.x);
         tape[3] = t4(s.h, F.y);
         tape[4] = t4(M, F.z);
@@ -161,13 +186,22 @@ template <typename T> VX_HD void diff_voxel_fwd(const DD<T> &d, int v, double tN
 template <typename T> VX_HD void diff_gather_adjoint(const DD<T> &d, int v, double tStep) {
     T4<T> au = d.au[v], aq = d.aq[v];
     T tb = au.w;
+    int vl[6];
+    T4<T> a[6], b[6];  // every link's words in flight at once, added in direction order
+#pragma unroll
+    for (int k = 0; k < 6; k++) vl[k] = d.vlinks[6 * v + k];
+#pragma unroll
     for (int k = 0; k < 6; k++) {
-        const int l = d.vlinks[6 * v + k];
-        if (l < 0) continue;
-        const T4<T> a = (k & 1) ? d.c2[l] : d.c0[l], b = (k & 1) ? d.c3[l] : d.c1[l];
-        au.x += a.x; au.y += a.y; au.z += a.z;
-        tb += a.w;
-        aq.x += b.x; aq.y += b.y; aq.z += b.z; aq.w += b.w;
+        if (vl[k] < 0) continue;
+        a[k] = (k & 1) ? d.c2[vl[k]] : d.c0[vl[k]];
+        b[k] = (k & 1) ? d.c3[vl[k]] : d.c1[vl[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        if (vl[k] < 0) continue;
+        au.x += a[k].x; au.y += a[k].y; au.z += a[k].z;
+        tb += a[k].w;
+        aq.x += b[k].x; aq.y += b[k].y; aq.z += b[k].z; aq.w += b[k].w;
     }
     T dTdPhase;
     (void)temp_at(d, v, tStep, &dTdPhase);
