@@ -130,8 +130,9 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
     // threads take links from the front and voxels from the back: the waves left
     // without a link in the last round are those with a voxel more, and in a tile
     // of few links the contact sums run in other waves than the links (they need
-    // no barrier between them)
-    int vt = NT - 1 - tid;
+    // no barrier between them).  An FP64 tile without collisions has neither, and
+    // steps 2 % faster with both from the front.
+    int vt = COL || sizeof(T) == 4 ? NT - 1 - tid : tid;
     const int4 info = tiles[blockIdx.x];  // robot begin, robot count, voxels, links
     const int nr = info.y, nv = info.z, nl = info.w;
 
@@ -189,6 +190,9 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
     // ---- owned links: static description and state in registers
     int lEnds[KL], lInfo[KL];  // neg | pos << 16 (tile indices); axis | robot slot << 2 | material << 9
     LinkState<T> ls[KL];
+    // the strain is an output only: collision tiles, short of registers, store it
+    // in a launch's last step
+    float lStrain[COL ? 1 : KL];
 #pragma unroll
     for (int k = 0; k < KL; k++) {
         const int ll = tid + k * NT;
@@ -205,6 +209,7 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
             ls[k].a2v = {s1.z, s1.w, s2.x};
             ls[k].maxStrain = (float)s2.y;
             ls[k].flags = (int)s2.z;
+            if constexpr (!COL) lStrain[k] = (float)s2.w;
         }
     }
     // ---- owned voxels
@@ -483,10 +488,12 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
         // registers) is otherwise kept over the steps and pushes state into scratch.
         // Without collisions there is room for the rest, and taking it apart again
         // costs 1.5 % of the step.
+        if constexpr (COL || sizeof(T) == 4) {
 #pragma unroll
-        for (int k = 0; k < KV; k++)
+            for (int k = 0; k < KV; k++)
 #pragma unroll
-            for (int d = 0; d < 3; d++) pin(vLinks[k][d]);
+                for (int d = 0; d < 3; d++) pin(vLinks[k][d]);
+        }
         if constexpr (COL) {
             pin(tid);
             pin(vt);
@@ -633,10 +640,8 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
             sForce[3][ll] = o.mN.x; sForce[4][ll] = o.mN.y; sForce[5][ll] = o.mN.z;
             sForce[6][ll] = o.fP.x; sForce[7][ll] = o.fP.y; sForce[8][ll] = o.fP.z;
             sForce[9][ll] = o.mP.x; sForce[10][ll] = o.mP.y; sForce[11][ll] = o.mP.z;
-            if (s == nsteps - 1) {  // the strain is an output only
-                const int j0 = tr.loffG[j] + (ll - tr.lpre[j]);
-                a.ls2[j0].w = (T)o.strain;
-            }
+            if constexpr (!COL) lStrain[k] = o.strain;
+            else if (s == nsteps - 1) a.ls2[tr.loffG[j] + (ll - tr.lpre[j])].w = (T)o.strain;
             if (o.strain > 100.0f) tr.divNow[j] = 1;
         }
         // ---- contact forces, from the poses and momenta entering the step
@@ -737,16 +742,20 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
         const int gl = tr.loffG[j] + (ll - tr.lpre[j]);
         a.ls0[gl] = T4<T>{ls[k].pos2.x, ls[k].pos2.y, ls[k].pos2.z, ls[k].a1v.x};
         a.ls1[gl] = T4<T>{ls[k].a1v.y, ls[k].a1v.z, ls[k].a2v.x, ls[k].a2v.y};
-        T *const l2 = &a.ls2[gl].x;  // (the strain is there already)
-        l2[0] = ls[k].a2v.z;
-        l2[1] = (T)ls[k].maxStrain;
-        l2[2] = (T)ls[k].flags;
-        if (tr.diverged[j] == 1 || (tr.diverged[j] == 0 && tr.divNow[j])) {
-            // a robot that stopped in this launch: its last update was not the
-            // launch's last step, the voxels are still where that update saw them
-            const LinkMat &lm = LDSMAT ? sLM[lInfo[k] >> 9] : a.lmats[lInfo[k] >> 9];
-            if (!lm.fixedBoth)
-                l2[3] = (T)(float)qdiv(ls[k].pos2.x, rest_length<T>(lm, (float)sPose[7][lEnds[k] & 0xffff], (float)sPose[7][lEnds[k] >> 16]));
+        if constexpr (!COL) {
+            a.ls2[gl] = T4<T>{ls[k].a2v.z, (T)ls[k].maxStrain, (T)ls[k].flags, (T)lStrain[k]};
+        } else {
+            T *const l2 = &a.ls2[gl].x;
+            l2[0] = ls[k].a2v.z;
+            l2[1] = (T)ls[k].maxStrain;
+            l2[2] = (T)ls[k].flags;
+            if (tr.diverged[j] == 1 || (tr.diverged[j] == 0 && tr.divNow[j])) {
+                // a robot that stopped in this launch: its last update was not the
+                // launch's last step, the voxels are still where that update saw them
+                const LinkMat &lm = LDSMAT ? sLM[lInfo[k] >> 9] : a.lmats[lInfo[k] >> 9];
+                if (!lm.fixedBoth)
+                    l2[3] = (T)(float)qdiv(ls[k].pos2.x, rest_length<T>(lm, (float)sPose[7][lEnds[k] & 0xffff], (float)sPose[7][lEnds[k] >> 16]));
+            }
         }
     }
 #pragma unroll
