@@ -22,6 +22,7 @@
 // whose force fields or attach conditions read the samples has them taken on
 // the device (k_cycle_sample), and the runner uses those.
 #include <algorithm>
+#include <charconv>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -117,6 +118,16 @@ void appendf(std::string &s, const char *fmt, ...) {
     }
 }
 
+// v as printf's "%.<digits>f" writes it, followed by a comma: to_chars gives the same
+// characters (the exact value, correctly rounded) in about a fifth of the time,
+// and a frame is mostly such numbers
+void append_fixed(std::string &s, double v, int digits) {
+    char buf[512];  // the largest double has 309 digits before the point
+    char *end = std::to_chars(buf, buf + sizeof(buf) - 1, v, std::chars_format::fixed, digits).ptr;
+    *end++ = ',';
+    s.append(buf, end);
+}
+
 // .history header (VX3_SimulationManager.cu:40-51)
 std::string history_header(const Model &m) {
     std::string s = "\n{{{setting}}}<rescale>0.001</rescale>\n";
@@ -168,10 +179,11 @@ std::string history_frame(const Model &m, long long j, double t, const double *p
     if (m.recordVoxel) {
         appendf(s, "<<<Step%lld Time:%f>>>", j, t);
         for (int v : voxels) {
-            appendf(s, "%.1f,%.1f,%.1f,", pos[3 * v] * vs, pos[3 * v + 1] * vs, pos[3 * v + 2] * vs);
+            for (int i = 0; i < 3; i++) append_fixed(s, pos[3 * v + i] * vs, 1);
             const double w = q[4 * v];
             const double angle = 2.0 * std::acos(w > 1 ? 1 : w) * 57.29577951308232;  // AngleDegrees
-            appendf(s, "%.1f,%.2f,%.2f,%.2f,", angle, q[4 * v + 1], q[4 * v + 2], q[4 * v + 3]);
+            append_fixed(s, angle, 1);
+            for (int i = 1; i < 4; i++) append_fixed(s, q[4 * v + i], 2);
             // cornerOffset(NNN) and cornerOffset(PPP) (VX3_Voxel.cu:147-159)
             const VoxelMat &vm = m.vmats[m.vmat[v]];
             const double half = 0.5 * (vm.nomSize * (double)(1 + temp[v] * vm.alphaCTE));
@@ -192,11 +204,12 @@ std::string history_frame(const Model &m, long long j, double t, const double *p
                     off[corner][i] = (float)(half * st);
                 }
             }
-            appendf(s, "%.1f,%.1f,%.1f,%.1f,%.1f,%.1f,", off[0][0] * vs, off[0][1] * vs, off[0][2] * vs, off[1][0] * vs,
-                    off[1][1] * vs, off[1][2] * vs);
-            appendf(s, "%d,", m.vpal[v]);
-            appendf(s, "%.1f,", signal ? signal[v] : 0.0);  // localSignal
-            s += ";";
+            for (int corner = 0; corner < 2; corner++)
+                for (int i = 0; i < 3; i++) append_fixed(s, off[corner][i] * vs, 1);
+            s += std::to_string(m.vpal[v]);
+            s += ',';
+            append_fixed(s, signal ? signal[v] : 0.0, 1);  // localSignal
+            s += ';';
         }
         s += "<<<>>>";
     }
@@ -204,16 +217,15 @@ std::string history_frame(const Model &m, long long j, double t, const double *p
         appendf(s, "|[[[%lld]]]", j);
         for (int l = 0; l < m.nl(); l++) {
             if (lrem && lrem[l]) continue;
-            const int a = m.lpos[l], b = m.lneg[l];
-            appendf(s, "%.4f,%.4f,%.4f,", pos[3 * a], pos[3 * a + 1], pos[3 * a + 2]);
-            appendf(s, "%.4f,%.4f,%.4f,", pos[3 * b], pos[3 * b + 1], pos[3 * b + 2]);
-            s += ";";
+            for (int end : {m.lpos[l], m.lneg[l]})
+                for (int i = 0; i < 3; i++) append_fixed(s, pos[3 * end + i], 4);
+            s += ';';
         }
         if (att)
             for (const int4 &l : *att) {
-                appendf(s, "%.4f,%.4f,%.4f,", pos[3 * l.y], pos[3 * l.y + 1], pos[3 * l.y + 2]);
-                appendf(s, "%.4f,%.4f,%.4f,", pos[3 * l.x], pos[3 * l.x + 1], pos[3 * l.x + 2]);
-                s += ";";
+                for (int end : {l.y, l.x})
+                    for (int i = 0; i < 3; i++) append_fixed(s, pos[3 * end + i], 4);
+                s += ';';
             }
         s += "[[[]]]";
     }
