@@ -1,0 +1,82 @@
+"""Candidate lists at the edges of their making: more records around a voxel than
+the queue of its lanes holds, more candidates than a list holds, voxel counts at
+the edges of a lane group, wave and workgroup.  The flat and plain modes list with
+a wave's lanes, the persistent mode with one lane a voxel; contacts, which are
+summed in the lists' order, come out the same bit for bit."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path[:0] = [os.path.join(ROOT, "voxcraft-sim_amd")]
+
+import vx3mi  # noqa: E402
+from vx3mi import configs  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def block_models(dims):
+    n = int(np.prod(dims))
+    prob = dict(configs.config0(), dims=dims, cells=np.ones(n, np.int8), phase=np.linspace(0, 1, n), enable_collision=1)
+    return [vx3mi.Model.from_problem(prob)] * 3
+
+
+def outcome(b):
+    return dict(b.state(), pairs=b.contact_pairs(), flags=b.voxel_flags(), diverged=b.diverged())
+
+
+def assert_same(a, b):
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims,squeeze", [((1, 1, 2), 0.7), ((4, 4, 1), 0.6), ((5, 5, 5), 0.72), ((9, 7, 1), 0.5), ((6, 6, 5), 0.5),
+                                          ((7, 6, 6), 0.3), ((12, 12, 12), 0.45)])
+def test_lists_of_lanes_equal_lists_of_one_lane(precision, dims, squeeze):
+    models = block_models(dims)
+    out = []
+    for mode in (vx3mi.MODE_PERSISTENT, vx3mi.MODE_FLAT, vx3mi.MODE_PLAIN):
+        b = vx3mi.Batch(models, precision)
+        for r in range(3):  # each robot its own jitter, so that they list at different steps
+            pos = b.state(r)["pos"]
+            c = pos.mean(axis=0)
+            b.set_state(r, pos=c + squeeze * (pos - c) + np.random.default_rng(r).normal(scale=3e-5 * r, size=pos.shape))
+        b.record_contacts()
+        for _ in range(6):
+            b.step(1, mode=mode)
+        out.append(outcome(b))
+        b.close()
+    assert_same(out[0], out[1])
+    assert_same(out[0], out[2])
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims,squeeze,speed", [((4, 4, 4), 1.0, 0.0), ((5, 5, 5), 0.72, 0.0), ((7, 6, 6), 0.5, 0.0), ((9, 5, 3), 1.0, 3.0),
+                                                ((6, 6, 5), 1.0, 30.0), ((20, 20, 12), 1.0, 3.0)])
+def test_listings_beside_the_steps_equal_listings_before_them(precision, dims, squeeze, speed):
+    """Calls of many flat steps start their listings some steps ahead; the plain
+    mode lists before the step that needs it.  speed (m/s, falling apart towards
+    the middle): voxels cross the skin of their lists within a few steps or one."""
+    models = block_models(dims)
+    out = []
+    for mode in (vx3mi.MODE_PLAIN, vx3mi.MODE_FLAT):
+        b = vx3mi.Batch(models, precision)
+        for r in range(3):
+            st = b.state(r)
+            pos, c = st["pos"], st["pos"].mean(axis=0)
+            mass = 1e6 * 0.01**3
+            rng = np.random.default_rng(r)
+            b.set_state(r, pos=c + squeeze * (pos - c) + rng.normal(scale=3e-5 * r, size=pos.shape),
+                        linmom=speed * r * mass * rng.normal(size=pos.shape))
+        b.record_contacts()
+        for n in (1, 90, 7, 8, 33):  # listings before each step and beside them in turn
+            b.step(n, mode=mode)
+        out.append(outcome(b))
+        listings = b.listings()
+        b.close()
+    assert_same(out[0], out[1])
+    assert (listings > 0).all()

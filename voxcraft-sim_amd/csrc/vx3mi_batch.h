@@ -73,6 +73,11 @@ struct RobotTime {
     double scom[3], shist[2][3];
     double recentAngle, closeness;
     int closePairs, angleSamples;
+    // listings beside the steps: per step parity the step whose contacts test every
+    // pair (the lists may miss one), and the step the last listing began
+    int hardStep[2];
+    int listStep;
+    int pad;
     int attachUsed;      // pool entries handed out so far (attach)
     int attachOverflow;  // a voxel had more attach candidates than it keeps (kAttachPerVoxel), or the pool ran out
 };

@@ -175,7 +175,17 @@ template <typename T> __device__ __forceinline__ void pin(T4<T> &x) {
     pin(x.w);
 }
 
-template <typename T> __device__ __forceinline__ void voxel_update(const Dev<T> &a, int v, int parity) {
+// gpu_update_cilia_force (VX3_VoxelyzeKernel.cu:846-858): surface voxels of a
+// cilia material once TurnOnCiliaAfterThisManySeconds has passed, with the
+// orientation q and the signal ls entering the step (t: its time)
+template <typename T> __device__ __forceinline__ V3<T> cilia_force(const VoxelCilia &c, double ls, bool surface, double t, Q4<T> q) {
+    if (!surface || c.coef == 0 || c.onAfter > t) return V3<T>{0, 0, 0};
+    const V3<T> b = {(T)(c.base[0] + ls * c.shift[0]), (T)(c.base[1] + ls * c.shift[1]), (T)(c.base[2] + ls * c.shift[2])};
+    return qrot(q, b) * (T)c.coef;
+}
+
+// LISTED: the caller keeps the robots' listing flags (listings beside the steps)
+template <bool LISTED = false, typename T> __device__ __forceinline__ void voxel_update(const Dev<T> &a, int v, int parity) {
     // the loads that need only v (and the link forces, once the link ids are in)
     // are issued before the robot's checks: each check returns early, and a load
     // after it would wait for the loads before it.  The values are pinned where
@@ -201,7 +211,7 @@ template <typename T> __device__ __forceinline__ void voxel_update(const Dev<T> 
         }
     }
     RobotTime *rt = a.rt + r;
-    {  // this step's listing flags: the lists are built and read by now
+    if constexpr (!LISTED) {  // this step's listing flags: the lists are built and read by now
         const RobotParams &rp = a.rp[r];
         if (v == rp.voff && rp.scount > 0 && rt->stale[parity]) {
             rt->listings += 1;
@@ -263,18 +273,7 @@ template <typename T> __device__ __forceinline__ void voxel_update(const Dev<T> 
         field = {f.x, f.y, f.z};
     }
     V3<T> cil = {0, 0, 0};
-    if (a.cilia) {
-        // gpu_update_cilia_force (VX3_VoxelyzeKernel.cu:846-858): surface voxels of a
-        // cilia material once TurnOnCiliaAfterThisManySeconds has passed, with the
-        // orientation and the signal entering the step
-        const VoxelCilia &c = a.cilia[v];
-        if (surface && c.coef != 0 && !(c.onAfter > rt->time[parity])) {
-            const double ls = a.sig ? a.sig[v].local : 0.0;  // localSignal
-            const V3<T> b = {(T)(c.base[0] + ls * c.shift[0]), (T)(c.base[1] + ls * c.shift[1]),
-                             (T)(c.base[2] + ls * c.shift[2])};
-            cil = qrot(s.q, b) * (T)c.coef;
-        }
-    }
+    if (a.cilia) cil = cilia_force(a.cilia[v], a.sig ? a.sig[v].local : 0.0, surface, rt->time[parity], s.q);
     voxel_step<T>(vm, a.exts, dt, a.lat[v], temp, fs, ms, contact, field, s, a.cilia ? &cil : nullptr);
     if (rp.varyTemp && !(vm.thermalOnAfter > tnext)) {
         if constexpr (std::is_same<T, float>::value)
@@ -286,7 +285,7 @@ template <typename T> __device__ __forceinline__ void voxel_update(const Dev<T> 
     a.pq1[v] = T4<T>{s.q.x, s.q.y, s.q.z, (T)temp};
     a.mo0[v] = T4<T>{s.p.x, s.p.y, s.p.z, s.h.x};
     a.mo1[v] = T4<T>{s.h.y, s.h.z, (T)s.flags, (T)0};
-    if (rp.collisions || rp.attach) col_track(a, v, s.u, rt, rp, parity);  // attach uses the candidate lists too
+    if (!LISTED && (rp.collisions || rp.attach)) col_track(a, v, s.u, rt, rp, parity);  // attach uses the candidate lists too
     // the voxel's own signal section ends a full timeStep (not one of a voxel
     // with all six degrees of freedom fixed, VX3_Voxel.cu:166-172)
     if (a.sig && rp.signals && dt != 0.0f && !(vm.ext >= 0 && a.exts[vm.ext].dof == DOF_ALL)) {
@@ -519,10 +518,9 @@ template <typename T> __device__ __forceinline__ void col_scatter(const Dev<T> &
 // around surface voxel s (voxel v), from the grid of the last listing; pw is
 // w's record of that listing (position field, lattice site), loaded with POS
 template <bool POS, typename T, typename F>
-__device__ __forceinline__ void col_grid_each(const Dev<T> &a, const RobotParams &rp, int s, int v, F &&f, int c0 = 0,
-                                              int cstep = 1) {
+__device__ __forceinline__ void col_grid_each(const Dev<T> &a, const RobotParams &rp, int s, int v, F &&f) {
     const int4 cs = a.scell[s];
-    for (int c = c0; c < 27; c += cstep) {  // the cells c0, c0 + cstep, ...
+    for (int c = 0; c < 27; c++) {
         const int cx = cs.x + c % 3 - 1, cy = cs.y + (c / 3) % 3 - 1, cz = cs.z + c / 9 - 1;
         const int key = (int)(cell_hash(cx, cy, cz) & (unsigned)rp.mask);
         const int b0 = a.cstart[rp.toff + key], b1 = a.cstart[rp.toff + key + 1];
@@ -543,20 +541,18 @@ __device__ __forceinline__ void col_grid_each(const Dev<T> &a, const RobotParams
 // can lose links or voxels (the contact phase tests the current links then);
 // more than kMaxCand: ccount = their number and the voxel searches the grid
 // itself
-// The candidates of surface voxel s (voxel v) in the cells c0, c0 + cstep, ...
-// of the 27, in ascending order into out[0 .. cap); returns their number (also
-// beyond cap).  out is global or LDS memory.
+// The candidates of surface voxel s (voxel v) in ascending order into
+// out[0 .. cap); returns their number (also beyond cap).
 template <typename T>
-__device__ __forceinline__ int col_list_cells(const Dev<T> &a, const RobotParams &rp, int s, int v, int c0, int cstep,
-                                              int *out, int cap) {
+__device__ __forceinline__ int col_list_cells(const Dev<T> &a, const RobotParams &rp, int s, int v, int *out, int cap) {
     const VoxelMat &mi = a.vmats[a.vmat[v]];
-    const T4<T> pv = a.pq0[v];
+    const T4<T> pv = a.bpos[v];  // both positions are those at the listing
     const int pkv = a.lat[v];
     const T L = (T)mi.nomSize, R = (T)rp.listR;
     int n = 0;
     col_grid_each<true>(
         a, rp, s, v,
-        [&](int w, const T4<T> &pw) {  // pw: w's position now
+        [&](int w, const T4<T> &pw) {  // pw: w's position
             const int3 o = lat_offset(pkv, word_lat<T>(pw.w));
             if (!rp.listLinked && col_linked(a, v, o.x, o.y, o.z)) return;
             if (mi.fixed && a.vmats[a.vmat[w]].fixed) return;
@@ -568,8 +564,7 @@ __device__ __forceinline__ int col_list_cells(const Dev<T> &a, const RobotParams
                 out[k] = w;
             }
             n++;
-        },
-        c0, cstep);
+        });
     return n;
 }
 template <typename T> __device__ __forceinline__ void col_list(const Dev<T> &a, int s, int parity) {
@@ -577,7 +572,7 @@ template <typename T> __device__ __forceinline__ void col_list(const Dev<T> &a, 
     const int r = a.vrob[v];
     const RobotTime *rt = a.rt + r;
     if (!rt->stale[parity] || rt->diverged) return;
-    a.ccount[s] = col_list_cells(a, a.rp[r], s, v, 0, 1, a.clist + (long)s * kMaxCand, kMaxCand);
+    a.ccount[s] = col_list_cells(a, a.rp[r], s, v, a.clist + (long)s * kMaxCand, kMaxCand);
 }
 
 // The contact force of surface voxel s from the partners inside its envelope,
@@ -586,80 +581,149 @@ template <typename T> __device__ __forceinline__ void col_list(const Dev<T> &a, 
 // hits, the forced signal, and the pair record when one is kept.  kContactLanes
 // consecutive work-items (lane 0..) share a voxel: each evaluates every
 // kContactLanes-th candidate, and the forces are added in list order.  LIST: in
-// a step whose listing passes have run (the grid is rebuilt), lane 0 builds the
-// voxel's candidate list first and then takes every candidate itself (the list
-// is its own writes; a listing comes every ~100 steps).  The voxel update of the
-// step clears the listing flags.
+// a step whose listing passes have run (the grid is rebuilt), the wave builds its
+// voxels' candidate lists first (every lane calls; there: the lane has a voxel; q:
+// LDS as col_list_wave's).  The voxel update of the step clears the listing flags.
 constexpr int kContactLanes = 4;
 
-// The list of surface voxel s (voxel v) built by its kContactLanes contact lanes
-// (lane = 0 ..; seg: kMaxCand ints of LDS for the voxel): lane j walks the cells
-// j, j + kContactLanes, ... into its part of seg, in ascending order; then each
-// lane ranks its candidates among all of them and writes them to their places
-// in the list row -- the list and count col_list makes.  When a lane finds more
-// than its part holds, lane 0 makes the whole list alone.  Returns the count to
-// every lane.
+// The list and count col_list makes, built by kListLanes consecutive lanes of a
+// wave for surface voxel s (voxel v; live: it has one to make; every lane of the
+// wave calls).  The lanes take the 27 cells side by side, put the records these
+// hold into a queue, take the records side by side, and rank what stays: four
+// dependent loads, where a lane that walks its share of the cells (the contact
+// phase's four lanes did) makes a chain of two for each cell and one for each
+// record: a listing step of one robot took 43 us of which a step is 9.
+// q: kListQueue ints of LDS, kMaxCand for the list and the rest for the queue;
+// more records than that, and one lane makes the whole list.
+constexpr int kListLanes = 16, kListQueue = 200;  // (a group's row starts 8 banks after the one before)
 template <typename T>
-__device__ __forceinline__ int col_list_lanes(const Dev<T> &a, const RobotParams &rp, int s, int v, int lane, int *seg) {
-    constexpr int PART = kMaxCand / kContactLanes;
-    int *list = a.clist + (long)s * kMaxCand;
-    const int own = col_list_cells(a, rp, s, v, lane, kContactLanes, seg + lane * PART, PART);
-    int cnt[kContactLanes], total = 0;
-    bool over = false;
+__device__ __forceinline__ int col_list_group(const Dev<T> &a, int s, int v, bool live, int *q) {
+    constexpr int NB = 3;
+    const int lane = threadIdx.x & (kListLanes - 1), base = threadIdx.x & 63 & ~(kListLanes - 1);
+    const RobotParams &rp = a.rp[a.vrob[v]];
+    const VoxelMat &mi = a.vmats[a.vmat[v]];
+    const int4 cs = a.scell[s];
+    const T4<T> pv = a.bpos[v];  // all positions are those at the listing
+    const int pkv = a.lat[v], l = a.vlinks[6 * v + min(lane, 5)];
+    const T L = (T)mi.nomSize, R = (T)rp.listR;
+    const int soff = rp.soff;
+    // direct links, to leave out
+    const unsigned linked = rp.listLinked ? 0 : (unsigned)(__ballot(l >= 0) >> base) & 63;
+    int b0[2], nb[2];
 #pragma unroll
-    for (int j = 0; j < kContactLanes; j++) {
-        cnt[j] = __shfl(own, j, kContactLanes);
-        total += cnt[j];
-        over |= cnt[j] > PART;
+    for (int j = 0; j < 2; j++) {
+        const int c = lane + j * kListLanes;
+        const int key = (int)(cell_hash(cs.x + c % 3 - 1, cs.y + (c / 3) % 3 - 1, cs.z + c / 9 - 1) & (unsigned)rp.mask);
+        b0[j] = a.cstart[rp.toff + key];
+        nb[j] = live && c < 27 ? a.cstart[rp.toff + key + 1] - b0[j] : 0;
     }
-    if (over) {  // the same for the voxel's lanes
-        if (lane == 0) total = col_list_cells(a, rp, s, v, 0, 1, list, kMaxCand);
-        total = __shfl(total, 0, kContactLanes);
-    } else {
-        __threadfence_block();  // the parts of the other lanes
-        for (int k = 0; k < own; k++) {
-            const int e = seg[lane * PART + k];
-            int rank = k;
+    int incl = nb[0] + nb[1];
+    for (int o = 1; o < kListLanes; o <<= 1) {
+        const int y = __shfl_up(incl, o, kListLanes);
+        if (lane >= o) incl += y;
+    }
+    const int total = __shfl(incl, kListLanes - 1, kListLanes);
+    const bool over = total > kListQueue - kMaxCand;
+    const int n0 = over ? 0 : total;
+    int *queue = q + kMaxCand, at = incl - nb[0] - nb[1];
 #pragma unroll
-            for (int j = 0; j < kContactLanes; j++) {
-                if (j == lane) continue;
-                for (int m = 0; m < cnt[j]; m++) rank += seg[j * PART + m] < e;
+    for (int j = 0; j < 2; j++)
+        for (int k = 0; k < (over ? 0 : nb[j]); k++) queue[at++] = (b0[j] + k) << 5 | (lane + j * kListLanes);
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses are carried out in order)
+    asm volatile("" ::: "memory");
+    int n = 0;
+    for (int k0 = 0; __any(k0 < n0); k0 += NB * kListLanes) {
+        int c[NB];
+        int4 g[NB];
+        T4<T> pw[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const int k = k0 + b * kListLanes + lane, e = k < n0 ? queue[k] : 0;
+            c[b] = k < n0 ? e & 31 : -1;
+            g[b] = a.grec[soff + (e >> 5)];
+            pw[b] = a.gpos[soff + (e >> 5)];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            // another cell of the bucket, itself
+            bool keep = c[b] >= 0 && g[b].x == cs.x + c[b] % 3 - 1 && g[b].y == cs.y + (c[b] / 3) % 3 - 1 &&
+                        g[b].z == cs.z + c[b] / 9 - 1 && g[b].w != v;
+            const int3 o = lat_offset(pkv, word_lat<T>(pw[b].w));
+            if (abs(o.x) + abs(o.y) + abs(o.z) == 1) {
+                const int d = o.x ? (o.x > 0 ? 0 : 1) : (o.y ? (o.y > 0 ? 2 : 3) : (o.z > 0 ? 4 : 5));
+                keep = keep && !(linked >> d & 1);
             }
-            list[rank] = e;
+            const V3<T> d = col_diff<T>(pv, pw[b], o, L);
+            keep = keep && !(d.x * d.x + d.y * d.y + d.z * d.z > R * R);
+            if (keep && mi.fixed) keep = !a.vmats[a.vmat[g[b].w]].fixed;
+            const unsigned m = (unsigned)(__ballot(keep) >> base) & ((1u << kListLanes) - 1);
+            const int to = n + __popc(m & ((1u << lane) - 1));
+            if (keep && to < kMaxCand) q[to] = g[b].w;
+            n += __popc(m);
         }
     }
-    if (lane == 0) a.ccount[s] = total;
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+    int *list = a.clist + (long)s * kMaxCand;
+    if (n <= kMaxCand)  // ascending: each to the place its rank among all gives it
+        for (int k = lane; k < n; k += kListLanes) {
+            const int e = q[k];
+            int rank = 0;
+#pragma unroll 4
+            for (int m = 0; m < n; m++) rank += q[m] < e;
+            list[rank] = e;
+        }
+    if (over) {
+        if (lane == 0) n = col_list_cells(a, rp, s, v, list, kMaxCand);
+        n = __shfl(n, 0, kListLanes);
+    }
+    if (live && lane == 0) a.ccount[s] = n;
     __threadfence_block();  // the list, for the other lanes
-    return total;
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");  // (the next group's queue comes after)
+    return n;
 }
 
-template <bool LIST, typename T> __device__ __forceinline__ void col_contact(const Dev<T> &a, int s, int parity, int lane, int *seg) {
-    // the loads that need only s or v are issued before the robot's checks (each
-    // returns early, and a load after it would wait for it): the voxel's pose,
-    // and its list as it stands with this lane's first candidate (a listing step
-    // rebuilds the list below, and lane 0 then reads it again)
-    const int v = a.surf[s];
-    const int ncPre = a.ccount[s];
-    const int *list = a.clist + (long)s * kMaxCand;
-    const int wFirst = list[lane];
-    const int r = a.vrob[v];
-    const int matI = a.vmat[v], pkv = a.lat[v];
-    const T4<T> qi0 = a.pq0[v], qi1 = a.pq1[v], mi0 = a.mo0[v];
-    RobotTime *rt = a.rt + r;
-    const RobotParams &rp = a.rp[r];
-    const bool listed = LIST && rt->stale[parity] && !rt->diverged;  // the same for the lanes of a voxel
-    const int nc = listed ? col_list_lanes(a, rp, s, v, lane, seg) : ncPre;
-    if (!rp.collisions || rt->diverged) return;
-    if (!col_active(a, v)) {
-        if (lane == 0) a.contactW[v] = T4<T>{0, 0, 0, 0};
-        return;
+// The lists of a wave's voxels, kContactLanes lanes each (every lane calls; want:
+// the voxel has one to make), four voxels at a time in kListRounds rounds, or the
+// rounds from r0 on only; returns the count to the voxel's lanes, nc to those with
+// nothing to make.
+constexpr int kListRounds = kListLanes / kContactLanes;
+template <typename T>
+__device__ __forceinline__ int col_list_wave(const Dev<T> &a, int s, int v, bool want, int nc, int r0, int rounds, int *q) {
+    const int me = threadIdx.x & 63, mine = me / kListLanes;
+#pragma unroll 1
+    for (int k = 0; k < kListRounds; k++) {
+        const bool now = want && mine == k && k >= r0 && k < r0 + rounds;
+        if (!__any(now)) continue;
+        const int from = k * kListLanes + mine * kContactLanes;
+        const int ts = __shfl(s, from), tv = __shfl(v, from);
+        const int n = col_list_group(a, ts, tv, __shfl((int)now, from) != 0, q);
+        const int got = __shfl(n, (me & (kListLanes - 1)) / kContactLanes * kListLanes);
+        if (now) nc = got;
     }
+    return nc;
+}
+
+// where the partners of a contact sum come from: the voxel's candidate list, the
+// grid of the last listing (more candidates than a list holds), or every surface
+// voxel of the robot (a listing beside the steps, when neither is known to hold them all)
+enum ColSource { COL_LIST, COL_GRID, COL_ALL };
+
+// the contact force on surface voxel v summed over its kContactLanes lanes (the
+// result is lane 0's), from the state a holds: the lanes take the candidates in
+// turn and add the forces in ascending partner order.  wFirst: this lane's first
+// candidate of a list.  hit: set when a target touches a non-target.
+template <typename T>
+__device__ __forceinline__ V3<T> col_contact_sum(const Dev<T> &a, const RobotParams &rp, RobotTime *rt, int s, int v, int lane,
+                                                 ColSource src, int nc, int wFirst, int matI, int pkv, const T4<T> &qi0,
+                                                 const T4<T> &qi1, const T4<T> &mi0, int &hit) {
+    const int *list = a.clist + (long)s * kMaxCand;
     const VoxelMat &mi = a.vmats[matI];
     const T L = (T)mi.nomSize;
     const T bsaI = base_size_average<T>(mi.nomSize, (float)qi1.w, mi.alphaCTE);
     const V3<T> velI = V3<T>{mi0.x, mi0.y, mi0.z} * (T)mi.massInv;
     const int ti = a.vtarget ? a.vtarget[v] : 0;
-    int hit = 0;
     // partner w when it is in contact now, its force in fw (links: whether to
     // test the current links; lists leave out linked neighbours unless the
     // robot can lose links)
@@ -693,9 +757,18 @@ template <bool LIST, typename T> __device__ __forceinline__ void col_contact(con
         return 1;
     };
     V3<T> f = {0, 0, 0};
-    if (nc <= kMaxCand) {
+    // adds one batch of the lanes' forces in list order
+    auto add = [&](int k0, int n, int in, const V3<T> &fk) {
+        for (int j = 0; j < kContactLanes && k0 + j < n; j++) {
+            const int inj = __shfl(in, j, kContactLanes);
+            const V3<T> fj = {__shfl(fk.x, j, kContactLanes), __shfl(fk.y, j, kContactLanes),
+                              __shfl(fk.z, j, kContactLanes)};
+            if (inj) f = f + fj;
+        }
+    };
+    if (src == COL_LIST) {
         const bool links = rp.listLinked != 0;
-        int w = listed ? list[lane] : wFirst;  // a listing step has just written the list
+        int w = wFirst;
         for (int k0 = 0; k0 < nc; k0 += kContactLanes) {
             const int kn = k0 + kContactLanes + lane;
             const int wn = kn < nc ? list[kn] : 0;  // the next batch in flight
@@ -703,18 +776,41 @@ template <bool LIST, typename T> __device__ __forceinline__ void col_contact(con
             int in = 0;
             if (k0 + lane < nc) in = partner(w, links, fk);
             w = wn;
-            for (int j = 0; j < kContactLanes && k0 + j < nc; j++) {  // list order
-                const int inj = __shfl(in, j, kContactLanes);
-                const V3<T> fj = {__shfl(fk.x, j, kContactLanes), __shfl(fk.y, j, kContactLanes),
-                                  __shfl(fk.z, j, kContactLanes)};
-                if (inj) f = f + fj;
+            add(k0, nc, in, fk);
+        }
+    } else if (src == COL_ALL) {
+        // four partners a lane in flight; whoever is not within the listing radius
+        // goes (the exact test's loads one by one: 12.6 ms for 12,000 voxels)
+        constexpr int NB = 4;
+        const T R2 = (T)rp.listR * (T)rp.listR;
+        for (int k0 = 0; k0 < rp.scount; k0 += NB * kContactLanes) {
+            int w[NB], pw[NB];
+            T4<T> qw[NB];
+            bool near[NB];
+#pragma unroll
+            for (int b = 0; b < NB; b++) w[b] = a.surf[rp.soff + min(k0 + b * kContactLanes + lane, rp.scount - 1)];
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                qw[b] = a.pq0[w[b]];
+                pw[b] = a.lat[w[b]];
+            }
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const V3<T> d = col_diff<T>(qi0, qw[b], lat_offset(pkv, pw[b]), L);
+                near[b] = k0 + b * kContactLanes + lane < rp.scount && w[b] != v && !(d.x * d.x + d.y * d.y + d.z * d.z > R2);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                if (!__any(near[b])) continue;
+                V3<T> fk = {0, 0, 0};
+                int in = 0;
+                if (near[b]) in = partner(w[b], true, fk);
+                add(k0 + b * kContactLanes, rp.scount, in, fk);
             }
         }
     } else if (lane == 0) {
         // more candidates than a list holds: ascending partners straight from the
-        // grid, which is rebuilt every step while this lasts
-        rt->stale[parity ^ 1] = 1;
-        if (a.anyStale) a.anyStale[parity ^ 1] = 1;
+        // grid
         int prev = -1;
         for (;;) {
             int next = INT_MAX;
@@ -728,9 +824,43 @@ template <bool LIST, typename T> __device__ __forceinline__ void col_contact(con
         }
     }
     for (int o = 1; o < kContactLanes; o <<= 1) hit |= __shfl_xor(hit, o, kContactLanes);
+    return f;
+}
+
+template <bool LIST, typename T>
+__device__ __forceinline__ void col_contact(const Dev<T> &a, int s, int parity, int lane, bool there = true, int *q = nullptr) {
+    // the loads that need only s or v are issued before the robot's checks (each
+    // returns early, and a load after it would wait for it): the voxel's pose,
+    // and its list as it stands with this lane's first candidate (a listing step
+    // rebuilds the list below, and lane 0 then reads it again)
+    const int v = a.surf[s];
+    const int ncPre = a.ccount[s];
+    const int *list = a.clist + (long)s * kMaxCand;
+    const int wFirst = list[lane];
+    const int r = a.vrob[v];
+    const int matI = a.vmat[v], pkv = a.lat[v];
+    const T4<T> qi0 = a.pq0[v], qi1 = a.pq1[v], mi0 = a.mo0[v];
+    RobotTime *rt = a.rt + r;
+    const RobotParams &rp = a.rp[r];
+    const bool listed = LIST && there && rt->stale[parity] && !rt->diverged;  // the same for the lanes of a voxel
+    int nc = ncPre;
+    if constexpr (LIST) nc = col_list_wave(a, s, v, listed, ncPre, 0, kListRounds, q);
+    if (!there || !rp.collisions || rt->diverged) return;
+    if (!col_active(a, v)) {
+        if (lane == 0) a.contactW[v] = T4<T>{0, 0, 0, 0};
+        return;
+    }
+    int hit = 0;
+    if (nc > kMaxCand && lane == 0) {  // searches the grid, which is rebuilt every step while this lasts
+        rt->stale[parity ^ 1] = 1;
+        if (a.anyStale) a.anyStale[parity ^ 1] = 1;
+    }
+    const V3<T> f = col_contact_sum(a, rp, rt, s, v, lane, nc <= kMaxCand ? COL_LIST : COL_GRID, nc,
+                                    listed ? list[lane] : wFirst,  // a listing step has just written the list
+                                    matI, pkv, qi0, qi1, mi0, hit);
     if (lane != 0) return;
     // with signals a non-target voxel touching a target receives a forced 100
-    if (hit && !ti && a.sig && rp.signals) {
+    if (hit && !(a.vtarget && a.vtarget[v]) && a.sig && rp.signals) {
         VoxelSignal sg = a.sig[v];
         signal_receive(sg, a.sigMat[v], 100, rt->time[parity], true);
         a.sig[v] = sg;
@@ -763,7 +893,7 @@ template <typename T> __device__ __forceinline__ void col_track(const Dev<T> &a,
 // per-voxel passes (the ranks inside a bucket may differ, which the ascending
 // lists do not see).
 constexpr int kCountPerGroup = 4096;  // four surface voxels per thread of a 1024-thread workgroup
-template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<T> &a, const RobotParams &rp, int s0, int s1) {
+template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<T> &a, const RobotParams &rp, int s0, int s1, T4<T> *old) {
     const double h = rp.listR;
     const int end = s1, nt = blockDim.x;
     for (int i0 = s0 + (int)threadIdx.x; i0 < end; i0 += 4 * nt) {
@@ -788,6 +918,7 @@ template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<
             const int key = (int)(cell_hash(cx, cy, cz) & (unsigned)rp.mask);
             a.scell[s] = int4{cx, cy, cz, key};
             a.srank[s] = atomicAdd(&a.ccnt[rp.toff + key], 1);
+            if (old) old[v[k]] = a.bpos[v[k]];
             a.bpos[v[k]] = q[k];
         }
     }
@@ -821,17 +952,14 @@ template <typename T> __device__ __forceinline__ void col_scatter_robot(const De
     }
 }
 
-// blockIdx.x: robot r0 + x; blockIdx.y: its part of the count pass
-template <typename T> __global__ __launch_bounds__(1024) void k_col_scan(Dev<T> a, int r0, int parity, int all) {
-    __shared__ int wsum[16];  // wave totals of col_scan
-    __shared__ int lastPart;
-    if (!all && !a.anyStale[parity]) return;
-    const int r = r0 + blockIdx.x;
-    const RobotParams &rp = a.rp[r];
-    if (!a.rt[r].stale[parity] || a.rt[r].diverged || rp.scount == 0) return;
-    const int parts = (rp.scount + kCountPerGroup - 1) / kCountPerGroup, part = blockIdx.y;
+// part of the grid of robot r (the calling workgroup's); old: where the positions
+// of the listing before are kept, if anywhere
+template <typename T>
+__device__ __forceinline__ void col_grid_part(const Dev<T> &a, const RobotParams &rp, int r, int part, int *wsum, int &lastPart,
+                                              T4<T> *old = nullptr) {
+    const int parts = (rp.scount + kCountPerGroup - 1) / kCountPerGroup;
     if (part >= parts) return;
-    col_count_robot(a, rp, rp.soff + part * kCountPerGroup, rp.soff + min(rp.scount, (part + 1) * kCountPerGroup));
+    col_count_robot(a, rp, rp.soff + part * kCountPerGroup, rp.soff + min(rp.scount, (part + 1) * kCountPerGroup), old);
     if (parts > 1) {
         // the workgroup that finishes its part last goes on with the whole
         // robot: every workgroup releases its cells, ranks and positions before
@@ -849,11 +977,22 @@ template <typename T> __global__ __launch_bounds__(1024) void k_col_scan(Dev<T> 
     __syncthreads();
     col_scatter_robot(a, rp);
 }
+
+// blockIdx.x: robot r0 + x; blockIdx.y: its part of the count pass
+template <typename T> __global__ __launch_bounds__(1024) void k_col_scan(Dev<T> a, int r0, int parity, int all) {
+    __shared__ int wsum[16];  // wave totals of col_scan
+    __shared__ int lastPart;
+    if (!all && !a.anyStale[parity]) return;
+    const int r = r0 + blockIdx.x;
+    const RobotParams &rp = a.rp[r];
+    if (!a.rt[r].stale[parity] || a.rt[r].diverged || rp.scount == 0) return;
+    col_grid_part(a, rp, r, blockIdx.y, wsum, lastPart);
+}
 template <typename T> __global__ __launch_bounds__(256) void k_col_contact(Dev<T> a, int s0, int n, int parity) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;  // kContactLanes per surface voxel
-    __shared__ int seg[256 / kContactLanes * kMaxCand];  // a listing step's parts of each voxel's list
-    if (i < n * kContactLanes)
-        col_contact<true>(a, s0 + i / kContactLanes, parity, i % kContactLanes, seg + threadIdx.x / kContactLanes * kMaxCand);
+    __shared__ int sQueue[256 / kListLanes * kListQueue];
+    const int k = i / kContactLanes;
+    col_contact<true>(a, s0 + min(k, n - 1), parity, i % kContactLanes, k < n, sQueue + threadIdx.x / kListLanes * kListQueue);
 }
 
 // the contact phase and the link updates of one step side by side in one launch
@@ -861,14 +1000,14 @@ template <typename T> __global__ __launch_bounds__(256) void k_col_contact(Dev<T
 // [0, nbl) update links, the rest compute contact forces
 template <typename T>
 __global__ __launch_bounds__(256) void k_contact_links(Dev<T> a, int nl, int nbl, int ns, int parity) {
-    __shared__ int seg[256 / kContactLanes * kMaxCand];  // a listing step's parts of each voxel's list
+    __shared__ int sQueue[256 / kListLanes * kListQueue];
     if ((int)blockIdx.x < nbl) {
         const int l = blockIdx.x * blockDim.x + threadIdx.x;
         if (l < nl) link_update(a, l, parity);
     } else {
         const int i = (blockIdx.x - nbl) * blockDim.x + threadIdx.x;
-        if (i < ns * kContactLanes)
-            col_contact<true>(a, i / kContactLanes, parity, i % kContactLanes, seg + threadIdx.x / kContactLanes * kMaxCand);
+        const int k = i / kContactLanes;
+        col_contact<true>(a, min(k, ns - 1), parity, i % kContactLanes, k < ns, sQueue + threadIdx.x / kListLanes * kListQueue);
     }
 }
 
@@ -1251,7 +1390,7 @@ template <typename T, int NT> __global__ __launch_bounds__(NT) void k_persistent
             }
             __syncthreads();
             for (int i = threadIdx.x; i < rp.scount * kContactLanes; i += NT)
-                col_contact<false>(a, rp.soff + i / kContactLanes, parity, i % kContactLanes, nullptr);  // listed above
+                col_contact<false>(a, rp.soff + i / kContactLanes, parity, i % kContactLanes);  // listed above
         }
         for (int l = rp.loff + threadIdx.x; l < rp.loff + rp.lcount; l += NT) link_update(a, l, parity);
         __syncthreads();
@@ -1262,6 +1401,7 @@ template <typename T, int NT> __global__ __launch_bounds__(NT) void k_persistent
 
 }  // namespace vx3mi
 #include "vx3mi_tile.h"
+#include "vx3mi_step.h"
 namespace vx3mi {
 
 // recommendedTimeStep (VX3_VoxelyzeKernel.cu:184-217) as a max-reduction:
@@ -1695,6 +1835,7 @@ template <typename T> struct Batch : BatchBase {
             }
         }
         S = (int)surf.size();
+        for (const RobotParams &p : hrp) largeRobot |= p.scount > kListYoungVoxels;
         tableBuckets = buckets;
         HIP_TRY(hipMemcpy(d_rp, hrp.data(), sizeof(RobotParams) * R, hipMemcpyHostToDevice));
         d.contact = nullptr;
@@ -1817,6 +1958,7 @@ template <typename T> struct Batch : BatchBase {
             d.sig = sd;
             d.sigMat = smd;
         }
+        if ((rc = listing_buffers())) return rc;
         return plan_tiles();
     }
 
@@ -1959,9 +2101,13 @@ template <typename T> struct Batch : BatchBase {
     // scatter; they return at once unless some robot's lists are stale (all:
     // check the robots' own flags only) -- the lists themselves are built by the
     // contact kernels that follow
-    void launch_listing(int r0, int nr, int parity, int all) {
-        int parts = 1;  // count-pass workgroups of the largest robot
+    int count_parts(int r0, int nr) const {  // count-pass workgroups of the largest robot
+        int parts = 1;
         for (int r = r0; r < r0 + nr; r++) parts = std::max(parts, (hrp[r].scount + kCountPerGroup - 1) / kCountPerGroup);
+        return parts;
+    }
+    void launch_listing(int r0, int nr, int parity, int all) {
+        const int parts = count_parts(r0, nr);
         k_col_scan<T><<<dim3(nr, parts), 1024, 0, stream>>>(d, r0, parity, all);
     }
     // the collision phase of one step for surface voxels [s0, s0 + n) (robots
@@ -1989,6 +2135,12 @@ template <typename T> struct Batch : BatchBase {
         if (anySignals) k_signal_deliver<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V);
         if (anyRemoval) k_removal<T><<<(d.nRemCand + 255) / 256, 256, 0, stream>>>(d, parity);
     }
+    ~Batch() override {
+        if (listHardHost) {
+            if (stream) (void)hipStreamSynchronize(stream);  // the last call may still write it
+            (void)hipHostFree(listHardHost);
+        }
+    }
     int kernels_per_flat_step() const {
         return 2 + (anyCollisions ? kCollisionLaunches - 1 : 0) + (anyForceField ? 1 : 0) + (anyRemoval ? 1 : 0) + (anySignals ? 1 : 0) +
                (anyDetach ? 1 : 0) + (anyAttach ? 3 : 0) + (anySample ? 1 : 0);
@@ -1998,6 +2150,70 @@ template <typename T> struct Batch : BatchBase {
     void launch_attach(int s0, int n, int r0, int nr) {
         if (n) k_attach_find<T><<<(n + 255) / 256, 256, 0, stream>>>(d, s0, n);
         k_attach_walk<T><<<nr, 256, 0, stream>>>(d, r0);
+    }
+
+    // ---- flat steps with listings beside them (vx3mi_step.h)
+    ListArgs<T> listing = {};
+    int *listHardHost = nullptr;
+    int gridParts = 1;
+    int listLast = 0, listRest = 0;    // steps of the last such call; calls left that list before each step
+    int young = kListYoung;            // steps left that a batch with large robots takes with a listing before each
+    bool largeRobot = false;
+    bool listBatch() const { return S > 0 && anyCollisions && !anyRemoval && !anyDetach && !anyAttach; }
+
+    int listing_buffers() {
+        if (!listBatch()) return VX3MI_OK;
+        int rc;
+        ListArgs<T> f{};
+        if ((rc = alloc(&f.hard, 2))) return rc;
+        HIP_TRY(hipHostMalloc((void **)&listHardHost, sizeof(int), hipHostMallocDefault));
+        *listHardHost = 0;
+        f.hardHost = listHardHost;
+        f.nmats = (int)hvmats.size();
+        gridParts = count_parts(0, R);
+        if ((rc = alloc(&f.bold, V))) return rc;
+        listing = f;
+        return VX3MI_OK;
+    }
+
+    // Whether a call's flat steps list beside them: enough steps to pay for the
+    // three launches around them, and not a batch whose robots kept crossing the
+    // skin of their lists faster than such a listing follows, so that their steps
+    // tested every pair (a step of that: 0.2 us for each voxel of the robot; more
+    // than 32 voxels' worth a step in the last call): that one lists before each
+    // step for a while.
+    static constexpr int kListMinSteps = 8;
+    bool list_beside(int nsteps) {
+        if (!listBatch() || nsteps < kListMinSteps) return false;
+        if (listRest > 0) { listRest--; return false; }
+        if (listLast > 0 && *listHardHost / 32 > listLast) {
+            *listHardHost = 0;
+            listRest = 15;
+            return false;
+        }
+        return true;
+    }
+
+    void launch_flat_step_listing(int k) {
+        ListArgs<T> f = listing;
+        f.step = k;
+        const int nbg = R * gridParts, nbl = (LP + 255) / 256, nbc = (S * kContactLanes + 255) / 256;
+        k_list_contact_links<T><<<nbg + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, LP, nbl, S, parity);
+        if (anyForceField) k_force_field<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V, parity);
+        k_list_voxels<T><<<(V + 255) / 256, 256, 0, stream>>>(d, f, V, parity);
+        if (anySample) k_cycle_sample<T><<<(R + 63) / 64, 64, 0, stream>>>(d, 0, R);
+        if (anySignals) k_signal_deliver<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V);
+        parity ^= 1;
+        launches += 2 + (anyForceField ? 1 : 0) + (anySample ? 1 : 0) + (anySignals ? 1 : 0);
+    }
+    int steps_listing(int nsteps) {
+        launch_listing(0, R, parity, 0);
+        k_list_begin<T><<<(S * kListLanes + 255) / 256, 256, 0, stream>>>(d, listing, R, S, parity);
+        for (int k = 0; k < nsteps; k++) launch_flat_step_listing(k);
+        k_list_end<T><<<R, 256, 0, stream>>>(d, listing, nsteps, parity);
+        listLast = nsteps;
+        launches += 3;
+        return VX3MI_OK;
     }
 
     int step(int nsteps, float dt, int mode) override {
@@ -2076,6 +2292,17 @@ template <typename T> struct Batch : BatchBase {
                 parity = (parity + k) & 1;
                 launches++;
             }
+        } else if (listBatch() && largeRobot && young > 0 && nsteps >= kListMinSteps) {
+            const int k = std::min(nsteps, young), rest = nsteps - k;
+            for (int s = 0; s < (rest >= kListMinSteps ? k : nsteps); s++) {
+                launch_flat_step(parity);
+                parity ^= 1;
+                launches += kernels_per_flat_step();
+            }
+            young -= k;
+            if (rest >= kListMinSteps && (rc = steps_listing(rest))) return rc;
+        } else if (list_beside(nsteps)) {
+            if ((rc = steps_listing(nsteps))) return rc;
         } else {
             // 1000-step graphs while at least that many steps remain, then 64-step
             // ones, then single steps
@@ -2174,6 +2401,7 @@ template <typename T> struct Batch : BatchBase {
     // the candidate lists of every robot are rebuilt by the next step (after the
     // state was replaced)
     int mark_stale() {
+        young = kListYoung;
         if (!anyCollisions) return VX3MI_OK;
         k_mark_stale<T><<<(R + 255) / 256, 256, 0, stream>>>(d_rt, R, d.anyStale);
         HIP_TRY(hipGetLastError());
