@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "vx3mi_batch.h"
+#include "vx3mi_stage.h"
 
 namespace vx3mi {
 
@@ -1958,8 +1959,8 @@ template <typename T> struct Batch : BatchBase {
             d.sig = sd;
             d.sigMat = smd;
         }
-        if ((rc = listing_buffers())) return rc;
-        return plan_tiles();
+        if ((rc = plan_tiles())) return rc;
+        return autoMode == VX3MI_MODE_FLAT ? listing_buffers() : VX3MI_OK;
     }
 
     // Longest-processing-time bin packing of robots into tiles (k_tile): at
@@ -2152,6 +2153,8 @@ template <typename T> struct Batch : BatchBase {
         k_attach_walk<T><<<nr, 256, 0, stream>>>(d, r0);
     }
 
+    Stage<T4<T>> stage;  // reading the state back
+
     // ---- flat steps with listings beside them (vx3mi_step.h)
     ListArgs<T> listing = {};
     int *listHardHost = nullptr;
@@ -2161,12 +2164,13 @@ template <typename T> struct Batch : BatchBase {
     bool largeRobot = false;
     bool listBatch() const { return S > 0 && anyCollisions && !anyRemoval && !anyDetach && !anyAttach; }
 
+    // with the batch where it steps flat by default, else on first use (0.1 ms)
     int listing_buffers() {
-        if (!listBatch()) return VX3MI_OK;
+        if (!listBatch() || listing.bold) return VX3MI_OK;
         int rc;
         ListArgs<T> f{};
         if ((rc = alloc(&f.hard, 2))) return rc;
-        HIP_TRY(hipHostMalloc((void **)&listHardHost, sizeof(int), hipHostMallocDefault));
+        if (!listHardHost) HIP_TRY(hipHostMalloc((void **)&listHardHost, sizeof(int), hipHostMallocDefault));
         *listHardHost = 0;
         f.hardHost = listHardHost;
         f.nmats = (int)hvmats.size();
@@ -2207,6 +2211,8 @@ template <typename T> struct Batch : BatchBase {
         launches += 2 + (anyForceField ? 1 : 0) + (anySample ? 1 : 0) + (anySignals ? 1 : 0);
     }
     int steps_listing(int nsteps) {
+        int rc = listing_buffers();
+        if (rc) return rc;
         launch_listing(0, R, parity, 0);
         k_list_begin<T><<<(S * kListLanes + 255) / 256, 256, 0, stream>>>(d, listing, R, S, parity);
         for (int k = 0; k < nsteps; k++) launch_flat_step_listing(k);
@@ -2352,25 +2358,34 @@ template <typename T> struct Batch : BatchBase {
         else { v0 = hrp[robot].voff; v1 = v0 + hrp[robot].vcount; }
     }
 
-    int get_state(int robot, double *pos, double *quat, double *lm, double *am) override {
-        std::vector<T4<T>> a0, a1, b0, b1;
-        int rc = fetch(a0, a1, b0, b1);
-        if (rc) return rc;
-        int v0, v1;
-        range(robot, v0, v1);
-        for (int v = v0; v < v1; v++) {
-            const int i = v - v0, pk = hlat[v];
+    // positions and orientations of m voxels from v0 on, from rows of pq0 and pq1
+    void unpack_pose(int v0, int m, const T4<T> *a0, const T4<T> *a1, double *pos, double *quat) const {
+        for (int i = 0; i < m; i++) {
+            const int v = v0 + i, pk = hlat[v];
             const double Ls = kAbsolutePositions<T> ? 0.0 : hvmats[hvmat[v]].nomSize;
             if (pos) {
-                pos[3 * i] = (pk & 1023) * Ls + (double)a0[v].x;
-                pos[3 * i + 1] = ((pk >> 10) & 1023) * Ls + (double)a0[v].y;
-                pos[3 * i + 2] = (pk >> 20) * Ls + (double)a0[v].z;
+                pos[3 * i] = (pk & 1023) * Ls + (double)a0[i].x;
+                pos[3 * i + 1] = ((pk >> 10) & 1023) * Ls + (double)a0[i].y;
+                pos[3 * i + 2] = (pk >> 20) * Ls + (double)a0[i].z;
             }
-            if (quat) { quat[4 * i] = a0[v].w; quat[4 * i + 1] = a1[v].x; quat[4 * i + 2] = a1[v].y; quat[4 * i + 3] = a1[v].z; }
-            if (lm) { lm[3 * i] = b0[v].x; lm[3 * i + 1] = b0[v].y; lm[3 * i + 2] = b0[v].z; }
-            if (am) { am[3 * i] = b0[v].w; am[3 * i + 1] = b1[v].x; am[3 * i + 2] = b1[v].y; }
+            if (quat) { quat[4 * i] = a0[i].w; quat[4 * i + 1] = a1[i].x; quat[4 * i + 2] = a1[i].y; quat[4 * i + 3] = a1[i].z; }
         }
-        return VX3MI_OK;
+    }
+
+    int get_state(int robot, double *pos, double *quat, double *lm, double *am) override {
+        int v0, v1;
+        range(robot, v0, v1);
+        const int n = v1 - v0;
+        return stage.read(stream, 4, {{d.pq0 + v0, d.pq1 + v0, d.mo0 + v0, d.mo1 + v0}, {n, n, n, n}},
+                          [&](int i0, int m, const T4<T> *at) {
+                              unpack_pose(v0 + i0, m, at, at + m, pos ? pos + 3 * (long)i0 : nullptr, quat ? quat + 4 * (long)i0 : nullptr);
+                              const T4<T> *b0 = at + 2 * m, *b1 = at + 3 * m;
+                              for (int k = 0; k < m; k++) {
+                                  const long i = i0 + k;
+                                  if (lm) { lm[3 * i] = b0[k].x; lm[3 * i + 1] = b0[k].y; lm[3 * i + 2] = b0[k].z; }
+                                  if (am) { am[3 * i] = b0[k].w; am[3 * i + 1] = b1[k].x; am[3 * i + 2] = b1[k].y; }
+                              }
+                          });
     }
 
     int set_state(int robot, const double *pos, const double *quat, const double *lm, const double *am) override {
@@ -2629,39 +2644,24 @@ template <typename T> struct Batch : BatchBase {
     int frame(int robot, double *pos, double *quat, float *temp, float *strain, float *maxStrain) override {
         if (robot < 0 || robot >= R) { set_error("robot index out of range"); return VX3MI_E_ARG; }
         const RobotParams &p = hrp[robot];
-        std::vector<T4<T>> a0((size_t)p.vcount), a1((size_t)p.vcount), l2((size_t)p.lcount);
-        HIP_TRY(hipStreamSynchronize(stream));
-        if (p.vcount) {
-            HIP_TRY(hipMemcpy(a0.data(), d.pq0 + p.voff, sizeof(T4<T>) * p.vcount, hipMemcpyDeviceToHost));
-            HIP_TRY(hipMemcpy(a1.data(), d.pq1 + p.voff, sizeof(T4<T>) * p.vcount, hipMemcpyDeviceToHost));
-        }
-        if (p.lcount) HIP_TRY(hipMemcpy(l2.data(), d.ls2 + p.loff, sizeof(T4<T>) * p.lcount, hipMemcpyDeviceToHost));
-        for (int i = 0; i < p.vcount; i++) {
-            const int v = p.voff + i, pk = hlat[v];
-            const double Ls = kAbsolutePositions<T> ? 0.0 : hvmats[hvmat[v]].nomSize;
-            if (pos) {
-                pos[3 * i] = (pk & 1023) * Ls + (double)a0[i].x;
-                pos[3 * i + 1] = ((pk >> 10) & 1023) * Ls + (double)a0[i].y;
-                pos[3 * i + 2] = (pk >> 20) * Ls + (double)a0[i].z;
-            }
-            if (quat) { quat[4 * i] = a0[i].w; quat[4 * i + 1] = a1[i].x; quat[4 * i + 2] = a1[i].y; quat[4 * i + 3] = a1[i].z; }
-            if (temp) temp[i] = (float)a1[i].w;
-        }
-        for (int l = 0; l < p.lcount; l++) {
-            if (strain) strain[l] = (float)l2[l].w;
-            if (maxStrain) maxStrain[l] = (float)l2[l].y;
-        }
-        return VX3MI_OK;
+        return stage.read(stream, 3, {{d.pq0 + p.voff, d.pq1 + p.voff, d.ls2 + p.loff}, {p.vcount, p.vcount, p.lcount}},
+                          [&](int i0, int m, const T4<T> *at) {
+                              const int nv = std::max(0, std::min(m, p.vcount - i0)), nl = std::max(0, std::min(m, p.lcount - i0));
+                              unpack_pose(p.voff + i0, nv, at, at + m, pos ? pos + 3 * (long)i0 : nullptr, quat ? quat + 4 * (long)i0 : nullptr);
+                              for (int i = 0; i < nv && temp; i++) temp[i0 + i] = (float)at[m + i].w;
+                              for (int l = 0; l < nl; l++) {
+                                  if (strain) strain[i0 + l] = (float)at[2 * m + l].w;
+                                  if (maxStrain) maxStrain[i0 + l] = (float)at[2 * m + l].y;
+                              }
+                          });
     }
 
     int get_flags(int robot, int *flags) override {
-        std::vector<T4<T>> a0, a1, b0, b1;
-        int rc = fetch(a0, a1, b0, b1);
-        if (rc) return rc;
         int v0, v1;
         range(robot, v0, v1);
-        for (int v = v0; v < v1; v++) flags[v - v0] = (int)b1[v].z;
-        return VX3MI_OK;
+        return stage.read(stream, 1, {{d.mo1 + v0}, {v1 - v0}}, [&](int i0, int m, const T4<T> *at) {
+            for (int i = 0; i < m; i++) flags[i0 + i] = (int)at[i].z;
+        });
     }
 
     int get_link_flags(int robot, int *flags, float *strain) override {

@@ -31,6 +31,7 @@
 #include "vx3mi_diff.h"
 #include "vx3mi_diff_batch.h"
 #include "vx3mi_diff_steps.h"
+#include "vx3mi_stage.h"
 
 namespace vx3mi {
 
@@ -445,6 +446,7 @@ template <typename T> struct DiffBatch : DiffBase {
         return VX3MI_OK;
     }
 
+    Stage<T4<T>> stage;  // reading the state back
     int get_state(int robot, double *pos, double *quat, double *lm, double *am) override {
         int v0 = 0, nv = V;
         if (robot >= 0) {
@@ -452,26 +454,25 @@ template <typename T> struct DiffBatch : DiffBase {
             v0 = hrp[robot].voff;
             nv = hrp[robot].vcount;
         }
-        std::vector<T4<T>> a((size_t)nv), b((size_t)nv), c((size_t)nv), e((size_t)nv);
         if (steps <= 0) { set_error("no forward run yet"); return VX3MI_E_ARG; }
-        HIP_TRY(hipStreamSynchronize(stream));
-        HIP_TRY(hipMemcpy(a.data(), fin + v0, sizeof(T4<T>) * nv, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(b.data(), fin + (size_t)V + v0, sizeof(T4<T>) * nv, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(c.data(), fin + (size_t)2 * V + v0, sizeof(T4<T>) * nv, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(e.data(), fin + (size_t)3 * V + v0, sizeof(T4<T>) * nv, hipMemcpyDeviceToHost));
-        for (int i = 0; i < nv; i++) {
-            const int v = v0 + i, pk = hlat[v];
-            const double Lv = hvm[v].nomSize;
-            if (pos) {
-                pos[3 * i] = (pk & 1023) * Lv + (double)a[i].x;
-                pos[3 * i + 1] = ((pk >> 10) & 1023) * Lv + (double)a[i].y;
-                pos[3 * i + 2] = (pk >> 20) * Lv + (double)a[i].z;
-            }
-            if (quat) { quat[4 * i] = b[i].x; quat[4 * i + 1] = b[i].y; quat[4 * i + 2] = b[i].z; quat[4 * i + 3] = b[i].w; }
-            if (lm) { lm[3 * i] = c[i].x; lm[3 * i + 1] = c[i].y; lm[3 * i + 2] = c[i].z; }
-            if (am) { am[3 * i] = e[i].x; am[3 * i + 1] = e[i].y; am[3 * i + 2] = e[i].z; }
-        }
-        return VX3MI_OK;
+        const T4<T> *at = fin + v0;
+        return stage.read(stream, 4, {{at, at + V, at + (size_t)2 * V, at + (size_t)3 * V}, {nv, nv, nv, nv}},
+                          [&](int i0, int m, const T4<T> *a) {
+                              const T4<T> *b = a + m, *c = b + m, *e = c + m;
+                              for (int k = 0; k < m; k++) {
+                                  const long i = i0 + k;
+                                  const int v = v0 + i0 + k, pk = hlat[v];
+                                  const double Lv = hvm[v].nomSize;
+                                  if (pos) {
+                                      pos[3 * i] = (pk & 1023) * Lv + (double)a[k].x;
+                                      pos[3 * i + 1] = ((pk >> 10) & 1023) * Lv + (double)a[k].y;
+                                      pos[3 * i + 2] = (pk >> 20) * Lv + (double)a[k].z;
+                                  }
+                                  if (quat) { quat[4 * i] = b[k].x; quat[4 * i + 1] = b[k].y; quat[4 * i + 2] = b[k].z; quat[4 * i + 3] = b[k].w; }
+                                  if (lm) { lm[3 * i] = c[k].x; lm[3 * i + 1] = c[k].y; lm[3 * i + 2] = c[k].z; }
+                                  if (am) { am[3 * i] = e[k].x; am[3 * i + 1] = e[k].y; am[3 * i + 2] = e[k].z; }
+                              }
+                          });
     }
 
     int backward(const double *gpos, const double *gquat, const double *glm, const double *gam, double *gphase,
