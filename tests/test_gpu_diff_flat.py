@@ -44,3 +44,28 @@ def test_flat_steps_equal_a_workgroup_per_robot(precision, dims, every, steps):
             assert np.array_equal(s[k], out[0][0][k]), k
         np.testing.assert_array_equal(gp, out[0][1])
         np.testing.assert_array_equal(ge, out[0][2])
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (4, 3, 3), (11, 9, 9)])
+def test_set_moduli_equal_the_models_own(precision, dims):
+    """The moduli of a model go through the host's constants, set ones through the
+    device's: the same bits in states and gradients."""
+    prob = configs.config3(seed=4, dims=dims)
+    n = prob["cells"].size
+    E = np.float32(10.0 ** np.random.default_rng(2).uniform(5, 8, size=n)).astype(np.float64)
+    own = vx3mi.Model.from_problem(dict(prob, voxel_E=E))
+    other = vx3mi.Model.from_problem(dict(prob, voxel_E=np.full(n, 3e6), phase=np.zeros(n)))
+    out = []
+    for m in (own, other):
+        d = vx3mi.Diff([m, m], precision)
+        if m is other:
+            d.set_params(np.tile(prob["phase"][prob["cells"] > 0], 2), np.tile(E[prob["cells"] > 0], 2))
+        d.forward(25)
+        out.append((d.state(), *d.backward(grad_pos=np.ones((d.nv, 3)))))
+        d.close()
+    (sa, pa, ea), (sb, pb, eb) = out
+    for k in sa:
+        assert np.array_equal(sa[k], sb[k]), k
+    np.testing.assert_array_equal(pa, pb)
+    np.testing.assert_array_equal(ea, eb)

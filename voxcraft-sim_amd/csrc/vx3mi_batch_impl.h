@@ -1981,8 +1981,8 @@ template <typename T> struct Batch : BatchBase {
         }
         int dev = 0, cus = 256;
         if (hipGetDevice(&dev) == hipSuccess) {
-            hipDeviceProp_t prop;
-            if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) cus = prop.multiProcessorCount;
+            int mp = 0;
+            if (hipDeviceGetAttribute(&mp, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && mp > 0) cus = mp;
         }
         const long slots = (long)cus * (SMALL ? 2 : 1);
         // A launch lasts as many rounds as its fullest workgroup slot runs tiles,

@@ -137,6 +137,23 @@ __global__ __launch_bounds__(256) void k_diff_rev_links(DD<T> d, int n, int segS
     diff_link_rev(d, l, n > 0 ? d.dt : (T)0, tapeV + ts * d.V * 5, tapeL + (ts * d.L + l) * 3);
 }
 
+// new moduli: what they set of the constants of voxel i and of link i (the rest stays
+// as it was laid out with the batch).  Bound by its loads, 12 us for 97,000 voxels;
+// the host's loop over them and the copy of all constants took 4.4 ms.
+template <typename T>
+__global__ __launch_bounds__(256) void k_diff_moduli(int V, int L, const DModulus *mod, const double *nom, const int2v *ends,
+                                                     const double *E, T *ET, DVox<T> *vc, DLink<T> *lc) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < V) {
+        ET[i] = (T)E[i];
+        diff_voxel_modulus(mod[i], E[i], vc[i]);
+    }
+    if (i < L) {
+        const int2v e = ends[i];
+        diff_link_modulus(E[e.x], E[e.y], nom[i], lc[i]);
+    }
+}
+
 template <typename T> __global__ __launch_bounds__(256) void k_diff_finish(DD<T> d, T *gE) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v < d.V) gE[v] = diff_finish_voxel(d, v);
@@ -159,7 +176,8 @@ template <typename T> struct DiffBatch : DiffBase {
     RobotParams *d_rp = nullptr;
     DVox<T> *d_vc = nullptr;
     DLink<T> *d_lc = nullptr;
-    double *d_phase = nullptr, *d_times = nullptr;
+    double *d_phase = nullptr, *d_times = nullptr, *d_nom = nullptr, *d_E64 = nullptr;
+    DModulus *d_mod = nullptr;
     T *d_E = nullptr, *d_gE = nullptr;
     T4<T> *ckV = nullptr, *ckL = nullptr, *tapeV = nullptr, *tapeL = nullptr;
     T4<T> *tapeV2 = nullptr, *tapeL2 = nullptr;  // second tape: recompute beside the reverse sweep
@@ -272,9 +290,9 @@ template <typename T> struct DiffBatch : DiffBase {
         constexpr bool f32 = std::is_same<T, float>::value;
         int maxLinks = 0, dev = 0, cus = 256;
         for (const RobotParams &p : hrp) maxLinks = std::max(maxLinks, p.lcount);
-        hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-            cus = prop.multiProcessorCount;
+        int mp = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&mp, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && mp > 0)
+            cus = mp;
         const double robot = ((f32 ? 12 : 21) + (f32 ? 0.0185 : 0.062) * maxLinks) * ((R + cus - 1) / cus);
         flatSteps = robot > (f32 ? 24 : 36) + (f32 ? 0.35e-3 : 0.9e-3) * V;
 
@@ -310,27 +328,53 @@ template <typename T> struct DiffBatch : DiffBase {
         d.al0 = arr[16]; d.al1 = arr[17]; d.al2 = arr[18];
         d.c0 = arr[19]; d.c1 = arr[20]; d.c2 = arr[21]; d.c3 = arr[22];
         d.gPhase = gph;
-        return set_params(hphase0.data(), hE0.data());
+        return init_params(hphase0.data(), hE0.data());
     }
 
-    int set_params(const double *phase, const double *E) override {
+    // the constants of the models' own moduli, and what set_params needs for others
+    int init_params(const double *phase, const double *E) {
         std::vector<DVox<T>> vc((size_t)V);
         std::vector<DLink<T>> lc((size_t)std::max(L, 1));
-        std::vector<T> Ev((size_t)V);
-        for (int v = 0; v < V; v++) {
+        // one block: a DModulus per voxel (three words), a length per link, then room
+        // for the moduli given to set_params
+        static_assert(sizeof(DModulus) == 3 * sizeof(double), "three words");
+        std::vector<double> laid((size_t)3 * V + L);
+        DModulus *mod = reinterpret_cast<DModulus *>(laid.data());
+        std::copy(hnom.begin(), hnom.end(), laid.begin() + (size_t)3 * V);
+        for (int v = 0; v < V; v++)
             if (!(E[v] > 0)) {
                 set_error("Young's modulus must be positive");
                 return VX3MI_E_ARG;
             }
-            Ev[v] = (T)E[v];
-        }
-        hphase.assign(phase, phase + V);
-        hE.assign(E, E + V);
+        for (int v = 0; v < V; v++) mod[v] = DModulus{hvm[v].mass, hvm[v].nomSize, hvm[v].zetaG, hvm[v].zetaC};
+        int rc;
+        double *block;
+        if ((rc = alloc(&block, (size_t)4 * V + L))) return rc;
+        d_mod = reinterpret_cast<DModulus *>(block);
+        d_nom = block + (size_t)3 * V;
+        d_E64 = d_nom + L;
         diff_constants<T>(hvm, hends.data(), haxis.data(), hnom.data(), hiz.data(), V, L, E, vc.data(), lc.data());
+        HIP_TRY(hipMemcpy(block, laid.data(), sizeof(double) * laid.size(), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(d_vc, vc.data(), sizeof(DVox<T>) * V, hipMemcpyHostToDevice));
         if (L) HIP_TRY(hipMemcpy(d_lc, lc.data(), sizeof(DLink<T>) * L, hipMemcpyHostToDevice));
+        std::vector<T> ET(E, E + V);
         HIP_TRY(hipMemcpy(d_phase, phase, sizeof(double) * V, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(d_E, Ev.data(), sizeof(T) * V, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(d_E, ET.data(), sizeof(T) * V, hipMemcpyHostToDevice));
+        steps = 0;
+        return VX3MI_OK;
+    }
+
+    int set_params(const double *phase, const double *E) override {
+        for (int v = 0; v < V; v++)
+            if (!(E[v] > 0)) {
+                set_error("Young's modulus must be positive");
+                return VX3MI_E_ARG;
+            }
+        HIP_TRY(hipMemcpyAsync(d_phase, phase, sizeof(double) * V, hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemcpyAsync(d_E64, E, sizeof(double) * V, hipMemcpyHostToDevice, stream));
+        k_diff_moduli<T><<<(std::max(V, L) + 255) / 256, 256, 0, stream>>>(V, L, d_mod, d_nom, d.lends, d_E64, d_E, d_vc, d_lc);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(stream));  // (the caller's arrays have been read)
         steps = 0;
         return VX3MI_OK;
     }
@@ -455,42 +499,55 @@ template <typename T> struct DiffBatch : DiffBase {
             nv = hrp[robot].vcount;
         }
         if (steps <= 0) { set_error("no forward run yet"); return VX3MI_E_ARG; }
-        const T4<T> *at = fin + v0;
-        return stage.read(stream, 4, {{at, at + V, at + (size_t)2 * V, at + (size_t)3 * V}, {nv, nv, nv, nv}},
-                          [&](int i0, int m, const T4<T> *a) {
-                              const T4<T> *b = a + m, *c = b + m, *e = c + m;
-                              for (int k = 0; k < m; k++) {
-                                  const long i = i0 + k;
-                                  const int v = v0 + i0 + k, pk = hlat[v];
-                                  const double Lv = hvm[v].nomSize;
-                                  if (pos) {
-                                      pos[3 * i] = (pk & 1023) * Lv + (double)a[k].x;
-                                      pos[3 * i + 1] = ((pk >> 10) & 1023) * Lv + (double)a[k].y;
-                                      pos[3 * i + 2] = (pk >> 20) * Lv + (double)a[k].z;
-                                  }
-                                  if (quat) { quat[4 * i] = b[k].x; quat[4 * i + 1] = b[k].y; quat[4 * i + 2] = b[k].z; quat[4 * i + 3] = b[k].w; }
-                                  if (lm) { lm[3 * i] = c[k].x; lm[3 * i + 1] = c[k].y; lm[3 * i + 2] = c[k].z; }
-                                  if (am) { am[3 * i] = e[k].x; am[3 * i + 1] = e[k].y; am[3 * i + 2] = e[k].z; }
-                              }
-                          });
+        double *const out[4] = {pos, quat, lm, am};
+        StageRows<T4<T>> rows{};
+        int K = 0, part[4];  // the arrays asked for, and where their rows come
+        for (int k = 0; k < 4; k++) {
+            part[k] = K;
+            if (!out[k]) continue;
+            rows.src[K] = fin + (size_t)k * V + v0;
+            rows.n[K++] = nv;
+        }
+        if (K == 0) return VX3MI_OK;
+        return stage.read(stream, K, rows, [&](int i0, int m, const T4<T> *at) {
+            const T4<T> *a = at + part[0] * m, *b = at + part[1] * m, *c = at + part[2] * m, *e = at + part[3] * m;
+            for (int k = 0; k < m; k++) {
+                const long i = i0 + k;
+                const int v = v0 + i0 + k, pk = hlat[v];
+                const double Lv = hvm[v].nomSize;
+                if (pos) {
+                    pos[3 * i] = (pk & 1023) * Lv + (double)a[k].x;
+                    pos[3 * i + 1] = ((pk >> 10) & 1023) * Lv + (double)a[k].y;
+                    pos[3 * i + 2] = (pk >> 20) * Lv + (double)a[k].z;
+                }
+                if (quat) { quat[4 * i] = b[k].x; quat[4 * i + 1] = b[k].y; quat[4 * i + 2] = b[k].z; quat[4 * i + 3] = b[k].w; }
+                if (lm) { lm[3 * i] = c[k].x; lm[3 * i + 1] = c[k].y; lm[3 * i + 2] = c[k].z; }
+                if (am) { am[3 * i] = e[k].x; am[3 * i + 1] = e[k].y; am[3 * i + 2] = e[k].z; }
+            }
+        });
     }
 
     int backward(const double *gpos, const double *gquat, const double *glm, const double *gam, double *gphase,
                  double *gE) override {
         if (steps <= 0) { set_error("backward needs a forward run first"); return VX3MI_E_ARG; }
         // adjoint of the final state
-        std::vector<T4<T>> au((size_t)V, T4<T>{0, 0, 0, 0}), aq = au, ap = au, ah = au;
-        for (int v = 0; v < V; v++) {
-            if (gpos) au[v] = T4<T>{(T)gpos[3 * v], (T)gpos[3 * v + 1], (T)gpos[3 * v + 2], 0};
-            if (gquat) aq[v] = T4<T>{(T)gquat[4 * v], (T)gquat[4 * v + 1], (T)gquat[4 * v + 2], (T)gquat[4 * v + 3]};
-            if (glm) ap[v] = T4<T>{(T)glm[3 * v], (T)glm[3 * v + 1], (T)glm[3 * v + 2], 0};
-            if (gam) ah[v] = T4<T>{(T)gam[3 * v], (T)gam[3 * v + 1], (T)gam[3 * v + 2], 0};
-        }
+        std::vector<T4<T>> up[4];
+        const double *src[4] = {gpos, gquat, glm, gam};
+        T4<T> *dst[4] = {d.au, d.aq, d.ap, d.ah};
+        for (int k = 0; k < 4; k++)
+            if (src[k]) {
+                up[k].resize((size_t)V);
+                const int w = k == 1 ? 4 : 3;
+                for (int v = 0; v < V; v++) {
+                    const double *g = src[k] + (long)w * v;
+                    up[k][v] = T4<T>{(T)g[0], (T)g[1], (T)g[2], w == 4 ? (T)g[3] : (T)0};
+                }
+            }
         HIP_TRY(hipEventRecord(ev0, stream));
-        HIP_TRY(hipMemcpyAsync(d.au, au.data(), sizeof(T4<T>) * V, hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipMemcpyAsync(d.aq, aq.data(), sizeof(T4<T>) * V, hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipMemcpyAsync(d.ap, ap.data(), sizeof(T4<T>) * V, hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipMemcpyAsync(d.ah, ah.data(), sizeof(T4<T>) * V, hipMemcpyHostToDevice, stream));
+        for (int k = 0; k < 4; k++) {
+            if (src[k]) HIP_TRY(hipMemcpyAsync(dst[k], up[k].data(), sizeof(T4<T>) * V, hipMemcpyHostToDevice, stream));
+            else HIP_TRY(hipMemsetAsync(dst[k], 0, sizeof(T4<T>) * V, stream));
+        }
         if (L) {
             HIP_TRY(hipMemsetAsync(d.al0, 0, sizeof(T4<T>) * L, stream));
             HIP_TRY(hipMemsetAsync(d.al1, 0, sizeof(T4<T>) * L, stream));

@@ -282,7 +282,33 @@ template <typename T> VX_HD T diff_finish_voxel(const DD<T> &d, int v) {
     return g;
 }
 
-// ---- host: per-voxel / per-link constants from the per-voxel moduli -------------
+// ---- per-voxel / per-link constants from the per-voxel moduli ----------------------
+// what a modulus sets: of a voxel (mass, nominal size, damping ratios, modulus) and
+// of a link (end moduli, nominal length), in double and then rounded to T; products,
+// quotients and square roots only, so that the host and the device agree bit for bit
+struct DModulus {
+    double mass, L;
+    float zetaG, zetaC;
+};
+template <typename T> VX_HD void diff_voxel_modulus(const DModulus &p, double E, DVox<T> &c) {
+    const double m = p.mass, Lv = p.L, I = m * Lv * Lv / 6.0;
+    c.gDampT = (T)(p.zetaG * 2.0 * sqrt(m * E * Lv));
+    c.gDampR = (T)(p.zetaG * 2.0 * sqrt(I * E * Lv * Lv * Lv));
+    c.cDampT = (T)(p.zetaC * 2.0 * sqrt(m * E * Lv));
+}
+template <typename T> VX_HD void diff_link_modulus(double Ea, double Eb, double Ll, DLink<T> &c) {
+    const double El = 2.0 * Ea * Eb / (Ea + Eb);
+    const double a2 = El * Ll * Ll * Ll / 12.0, b1 = El * Ll, b2 = El * Ll * Ll / 2.0, b3 = El * Ll * Ll * Ll / 6.0;
+    c.E = (T)El;
+    c.a2 = (T)a2; c.b1 = (T)b1; c.b2 = (T)b2; c.b3 = (T)b3;
+    c.sqA1 = (T)sqrt(El * Ll);
+    c.sqA2xIp = (T)sqrt(a2 * Ll * Ll / 6.0);
+    c.sqB1 = (T)sqrt(b1);
+    c.sqB2xFMp = (T)sqrt(b2 * Ll / 2.0);
+    c.sqB3xIp = (T)sqrt(b3 * Ll * Ll / 6.0);
+}
+
+// host: all of them
 // vm: material of each voxel; ends/axis/nom: link ends, axis, nominal length;
 // iz: lattice z of each voxel.  Constants in double, then rounded to T.
 template <typename T, typename VM>
@@ -294,9 +320,7 @@ inline void diff_constants(const VM &vm, const int2v *ends, const int *axis, con
         DVox<T> &c = vc[v];
         c.mInv = (T)(1.0 / m);
         c.IInv = (T)(1.0 / I);
-        c.gDampT = (T)(mt.zetaG * 2.0 * sqrt(m * E[v] * Lv));
-        c.gDampR = (T)(mt.zetaG * 2.0 * sqrt(I * E[v] * Lv * Lv * Lv));
-        c.cDampT = (T)(mt.zetaC * 2.0 * sqrt(m * E[v] * Lv));
+        diff_voxel_modulus(DModulus{m, Lv, mt.zetaG, mt.zetaC}, E[v], c);
         c.grav = (T)mt.gravF;
         c.L = (T)Lv;
         c.alpha = (T)mt.alphaCTE;
@@ -307,16 +331,9 @@ inline void diff_constants(const VM &vm, const int2v *ends, const int *axis, con
     }
     for (int l = 0; l < L; l++) {
         const int a = ends[l].x, b = ends[l].y;
-        const double Ea = E[a], Eb = E[b], El = 2.0 * Ea * Eb / (Ea + Eb), Ll = nom[l];
+        const double Ll = nom[l];
         DLink<T> &c = lc[l];
-        const double a2 = El * Ll * Ll * Ll / 12.0, b1 = El * Ll, b2 = El * Ll * Ll / 2.0, b3 = El * Ll * Ll * Ll / 6.0;
-        c.E = (T)El;
-        c.a2 = (T)a2; c.b1 = (T)b1; c.b2 = (T)b2; c.b3 = (T)b3;
-        c.sqA1 = (T)sqrt(El * Ll);
-        c.sqA2xIp = (T)sqrt(a2 * Ll * Ll / 6.0);
-        c.sqB1 = (T)sqrt(b1);
-        c.sqB2xFMp = (T)sqrt(b2 * Ll / 2.0);
-        c.sqB3xIp = (T)sqrt(b3 * Ll * Ll / 6.0);
+        diff_link_modulus(E[a], E[b], Ll, c);
         c.tArea = (T)(Ll * Ll);
         c.L = (T)Ll;
         c.nomN = (T)vm[a].nomSize;

@@ -34,13 +34,20 @@ template <typename W> class Stage {
     static constexpr int kRows = 16384;  // of all arrays together, per buffer (two of 256 KB or 512 KB)
     std::mutex lock;
     W *host = nullptr;
+    int rowsHeld = 0;
     hipEvent_t done[2] = {};
 
-    int ready() {  // on first use
-        if (host) return VX3MI_OK;
+    // room for the rows of a read, one buffer or two, kept for the next (pinning
+    // 1 MB takes 0.13 ms: a small batch holds what it needs)
+    int ready(int need) {
         for (hipEvent_t &e : done)
             if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        HIP_TRY(hipHostMalloc((void **)&host, sizeof(W) * 2 * kRows, hipHostMallocDefault));
+        if (need <= rowsHeld) return VX3MI_OK;
+        if (host) HIP_TRY(hipHostFree(host));
+        host = nullptr;
+        rowsHeld = 0;
+        HIP_TRY(hipHostMalloc((void **)&host, sizeof(W) * need, hipHostMallocDefault));
+        rowsHeld = need;
         return VX3MI_OK;
     }
 
@@ -65,9 +72,9 @@ public:
             HIP_TRY(hipStreamSynchronize(stream));
             return VX3MI_OK;
         }
-        int rc = ready();
-        if (rc) return rc;
         const int chunk = kRows / K;
+        int rc = ready(n <= chunk ? K * n : 2 * kRows);
+        if (rc) return rc;
         auto send = [&](int i0, int buf) -> int {
             const int m = n - i0 < chunk ? n - i0 : chunk;
             k_stage<W><<<dim3((m + 255) / 256, K), 256, 0, stream>>>(rows, i0, m, host + buf * kRows);

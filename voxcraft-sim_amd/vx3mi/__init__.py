@@ -607,6 +607,11 @@ class Diff:
         _check(lib().vx3mi_diff_get_state(self._h, int(robot), *[_ptr(a, C.c_double) for a in (pos, q, lm, am)]))
         return dict(pos=pos, quat=q, linmom=lm, angmom=am)
 
+    def _positions(self) -> np.ndarray:
+        pos = np.zeros((self.nv, 3))
+        _check(lib().vx3mi_diff_get_state(self._h, -1, _ptr(pos, C.c_double), None, None, None))
+        return pos
+
     def backward(self, grad_pos=None, grad_quat=None, grad_linmom=None, grad_angmom=None):
         """dL/dphase (per cycle) and dL/dE per voxel from dL/d(final state)."""
         g = [None if a is None else np.ascontiguousarray(a, dtype=np.float64).reshape(-1)

@@ -22,7 +22,7 @@ class _Simulate(torch.autograd.Function):
         ctx.diff = diff
         ctx.devices = (phase.device, E.device)
         ctx.dtypes = (phase.dtype, E.dtype)
-        return torch.from_numpy(diff.state()["pos"]).to(phase.device)
+        return torch.from_numpy(diff._positions()).to(phase.device)
 
     @staticmethod
     def backward(ctx, grad_pos: torch.Tensor):
