@@ -80,3 +80,29 @@ def test_listings_beside_the_steps_equal_listings_before_them(precision, dims, s
         b.close()
     assert_same(out[0], out[1])
     assert (listings > 0).all()
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("var", ["t", "hit"])
+def test_force_fields_of_long_calls_equal_the_plain_mode(precision, var):
+    """Fields beside the contacts, and after them where they read the collision
+    count: squeezed blocks of two materials, one of them a target, so that hits come."""
+    n = 60
+    base = configs.config0()
+    soft = base["materials"][0]
+    prob = dict(base, dims=(5, 4, 3), cells=(np.arange(n) % 2 + 1).astype(np.int8), phase=np.linspace(0, 1, n), enable_collision=1,
+                materials=[soft, dict(soft, is_target=1)],
+                force_field={"x": ("mtMUL", ("mtCONST", 1e-3), ("mtVAR", var)), "z": ("mtCONST", 1e-3)})
+    models = [vx3mi.Model.from_problem(prob)] * 2 + block_models((4, 3, 3))[:1]
+    out = []
+    for mode in (vx3mi.MODE_PLAIN, vx3mi.MODE_FLAT):
+        b = vx3mi.Batch(models, precision)
+        pos = b.state(0)["pos"]
+        c = pos.mean(axis=0)
+        b.set_state(0, pos=c + 0.6 * (pos - c))
+        for k in (3, 40):
+            b.step(k, mode=mode)
+        out.append(dict(b.state(), hits=b.hits()))
+        b.close()
+    assert out[0]["hits"][0] > 0
+    assert_same(*out)

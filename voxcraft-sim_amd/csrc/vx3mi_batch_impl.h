@@ -320,9 +320,7 @@ template <typename T> __global__ __launch_bounds__(256) void k_signal_deliver(De
 // The force-field force of each voxel for the coming voxel update, from the
 // position entering the step and the time before it (a kernel of its own: the
 // formula evaluator stays out of the update kernels).
-template <typename T> __global__ __launch_bounds__(256) void k_force_field(Dev<T> a, int v0, int nv, int parity) {
-    const int v = v0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= v0 + nv) return;
+template <typename T> __device__ __forceinline__ void field_update(const Dev<T> &a, int v, int parity) {
     const int r = a.vrob[v];
     const RobotParams &rp = a.rp[r];
     const RobotTime *rt = a.rt + r;
@@ -334,6 +332,10 @@ template <typename T> __global__ __launch_bounds__(256) void k_force_field(Dev<T
                            rt->recentAngle, rt->closeness, rt->closePairs);
     }
     a.field[v] = T4<T>{f.x, f.y, f.z, (T)0};
+}
+template <typename T> __global__ __launch_bounds__(256) void k_force_field(Dev<T> a, int v0, int nv, int parity) {
+    const int v = v0 + blockIdx.x * blockDim.x + threadIdx.x;
+    if (v < v0 + nv) field_update(a, v, parity);
 }
 
 // ---- collisions: candidate lists from a counting-sort grid --------------------
@@ -1488,6 +1490,7 @@ template <typename T> struct Batch : BatchBase {
     bool anyForceField = false;   // some robot has a force field (plain and flat modes only)
     bool anyCilia = false;        // some robot has EnableCilia (not in the tiles)
     bool anySignals = false;      // some robot has EnableSignals
+    bool anyFieldHit = false;     // some robot's force field reads the collision count
     bool anySample = false;       // some robot's formulas read the CycleStep samples (angle, closeness, pairs)
     // plain and flat modes only: force fields (their own kernel), removal and
     // signals (kernels between steps)
@@ -1589,6 +1592,7 @@ template <typename T> struct Batch : BatchBase {
             const unsigned sampledVars = (1u << MV_ANGLE) | (1u << MV_CLOSENESS) | (1u << MV_PAIRS);
             unsigned used = 0;
             for (int ax = 0; ax < 3; ax++) used |= mt_vars_used(m.forceField[ax]);
+            if (used & (1u << MV_HIT)) anyFieldHit = true;
             for (int k = 0; p.attach && k < 5; k++) used |= mt_vars_used(m.attachCond[k]);
             p.sample = (used & sampledVars) ? 1 : 0;
             p.pairR = m.maxDistPairs * m.latticeDim;
@@ -2202,13 +2206,24 @@ template <typename T> struct Batch : BatchBase {
         ListArgs<T> f = listing;
         f.step = k;
         const int nbg = R * gridParts, nbl = (LP + 255) / 256, nbc = (S * kContactLanes + 255) / 256;
-        k_list_contact_links<T><<<nbg + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, LP, nbl, S, parity);
-        if (anyForceField) k_force_field<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V, parity);
+        // Force fields beside the contacts: the evaluator's registers leave that launch
+        // one wave a SIMD, which a batch that does not fill the device does not notice
+        // (us a step with the field beside and after: 1,062 voxels 19.9 and 26.8 in
+        // FP32, 24.1 and 31.2 in FP64; 55,500 voxels 63.8 and 64.4, 76.5 and 77.1;
+        // 214,000 voxels 132.2 and 132.5, 175.4 and 171.6).  A field that reads the
+        // collision count comes after the contacts that add to it.
+        const bool beside = anyForceField && !anyFieldHit && V < 100000;
+        if (beside) {
+            const int nbf = (V + 255) / 256;
+            k_list_contact_links<T, 1><<<nbg + nbf + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, V, nbf, LP, nbl, S, parity);
+        } else
+            k_list_contact_links<T, 0><<<nbg + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, 0, 0, LP, nbl, S, parity);
+        if (anyForceField && !beside) k_force_field<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V, parity);
         k_list_voxels<T><<<(V + 255) / 256, 256, 0, stream>>>(d, f, V, parity);
         if (anySample) k_cycle_sample<T><<<(R + 63) / 64, 64, 0, stream>>>(d, 0, R);
         if (anySignals) k_signal_deliver<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V);
         parity ^= 1;
-        launches += 2 + (anyForceField ? 1 : 0) + (anySample ? 1 : 0) + (anySignals ? 1 : 0);
+        launches += 2 + (anyForceField && !beside ? 1 : 0) + (anySample ? 1 : 0) + (anySignals ? 1 : 0);
     }
     int steps_listing(int nsteps) {
         int rc = listing_buffers();

@@ -203,9 +203,11 @@ __device__ __forceinline__ void step_contact(const Dev<T> &a, const ListArgs<T> 
 }
 
 // the contact phase and the link updates of a step side by side in one launch (as
-// k_contact_links)
-template <typename T>
-__global__ __launch_bounds__(256) void k_list_contact_links(Dev<T> a, ListArgs<T> f, int nbg, int parts, int nl, int nbl, int ns, int parity) {
+// k_contact_links), the grids of robots that begin a listing, and with FIELD the
+// force fields (7 us as a launch of their own, formula by formula in each voxel)
+template <typename T, int FIELD>
+__global__ __launch_bounds__(256) void k_list_contact_links(Dev<T> a, ListArgs<T> f, int nbg, int parts, int nv, int nbf, int nl,
+                                                            int nbl, int ns, int parity) {
     __shared__ int sQueue[256 / kListLanes * kListQueue];
     __shared__ unsigned char sOwner[256];
     __shared__ float2 sEnv[4][kStepMats];
@@ -215,7 +217,10 @@ __global__ __launch_bounds__(256) void k_list_contact_links(Dev<T> a, ListArgs<T
         const int r = blk / parts;
         // (not the robot's diverged: a link of this launch may set it)
         if (a.rt[r].listStep == f.step) col_grid_part(a, a.rp[r], r, blk % parts, wsum, lastPart, f.bold);
-    } else if ((blk -= nbg) < nbl) {
+    } else if (FIELD && (blk -= nbg) < nbf) {
+        const int v = blk * blockDim.x + threadIdx.x;
+        if (v < nv) field_update(a, v, parity);
+    } else if ((blk -= FIELD ? nbf : nbg) < nbl) {
         const int l = blk * blockDim.x + threadIdx.x;
         if (l < nl) link_update(a, l, parity);
     } else {
