@@ -35,7 +35,7 @@ extern "C" {
 #define VX3MI_FP64 64
 
 /* step modes (vx3mi_step) */
-#define VX3MI_MODE_AUTO 0        /* tiled if possible, else persistent for small robots, else flat */
+#define VX3MI_MODE_AUTO 0        /* tiled where every robot fits a tile and that costs less, else flat; see vx3mi_batch_autotune */
 #define VX3MI_MODE_PLAIN 1       /* one robot per launch sequence (reference-style) */
 #define VX3MI_MODE_FLAT 2        /* one link launch + one voxel launch per step for the whole batch */
 #define VX3MI_MODE_PERSISTENT 3  /* one workgroup per robot, many steps per launch */
