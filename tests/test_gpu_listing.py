@@ -106,3 +106,25 @@ def test_force_fields_of_long_calls_equal_the_plain_mode(precision, var):
         b.close()
     assert out[0]["hits"][0] > 0
     assert_same(*out)
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("calls", [[(vx3mi.MODE_FLAT, 8), (vx3mi.MODE_PERSISTENT, 1), (vx3mi.MODE_PERSISTENT, 8), (vx3mi.MODE_FLAT, 7)],
+                                   [(vx3mi.MODE_TILED, 9), (vx3mi.MODE_PERSISTENT, 8), (vx3mi.MODE_FLAT, 20), (vx3mi.MODE_TILED, 7)]])
+def test_modes_in_turn_equal_the_plain_mode(precision, calls):
+    """Robots of different speeds whose lists are stale at the end of a call list
+    in the first step of the next, whichever mode it takes."""
+    models = block_models((7, 6, 6))
+    out = []
+    for plain in (True, False):
+        b = vx3mi.Batch(models, precision)
+        for r in range(3):
+            pos = b.state(r)["pos"]
+            c, rng = pos.mean(axis=0), np.random.default_rng(r)
+            b.set_state(r, pos=c + 0.5 * (pos - c) + rng.normal(scale=3e-5 * r, size=pos.shape),
+                        linmom=0.5 * r * rng.normal(size=pos.shape))
+        for mode, n in calls:
+            b.step(n, mode=vx3mi.MODE_PLAIN if plain else mode)
+        out.append(dict(b.state(), flags=b.voxel_flags(), diverged=b.diverged()))
+        b.close()
+    assert_same(*out)

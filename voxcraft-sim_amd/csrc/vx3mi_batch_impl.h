@@ -1400,6 +1400,9 @@ template <typename T, int NT> __global__ __launch_bounds__(NT) void k_persistent
         for (int v = rp.voff + threadIdx.x; v < rp.voff + rp.vcount; v += NT) voxel_update(a, v, parity);
         __syncthreads();
     }
+    // the first robot's voxel updates empty the batch's flags, also those that a robot
+    // some steps ahead has raised for the step after the launch
+    if (r == 0 && threadIdx.x == 0 && a.anyStale) a.anyStale[0] = a.anyStale[1] = 1;
 }
 
 }  // namespace vx3mi
