@@ -39,9 +39,9 @@ template <typename W> class Stage {
 
     // room for the rows of a read, one buffer or two, kept for the next (pinning
     // 1 MB takes 0.13 ms: a small batch holds what it needs)
-    int ready(int need) {
+    int ready(int need, bool chunks) {
         for (hipEvent_t &e : done)
-            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            if (chunks && !e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         if (need <= rowsHeld) return VX3MI_OK;
         if (host) HIP_TRY(hipHostFree(host));
         host = nullptr;
@@ -73,13 +73,14 @@ public:
             return VX3MI_OK;
         }
         const int chunk = kRows / K;
-        int rc = ready(n <= chunk ? K * n : 2 * kRows);
+        const bool chunks = n > chunk;
+        int rc = ready(chunks ? 2 * kRows : K * n, chunks);
         if (rc) return rc;
         auto send = [&](int i0, int buf) -> int {
             const int m = n - i0 < chunk ? n - i0 : chunk;
             k_stage<W><<<dim3((m + 255) / 256, K), 256, 0, stream>>>(rows, i0, m, host + buf * kRows);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipEventRecord(done[buf], stream));
+            if (chunks) HIP_TRY(hipEventRecord(done[buf], stream));
             return VX3MI_OK;
         };
         if ((rc = send(0, 0))) return rc;
@@ -89,7 +90,8 @@ public:
                 (void)hipStreamSynchronize(stream);
                 return rc;
             }
-            HIP_TRY(hipEventSynchronize(done[buf]));
+            if (chunks) HIP_TRY(hipEventSynchronize(done[buf]));
+            else HIP_TRY(hipStreamSynchronize(stream));
             unpack(i0, n - i0 < chunk ? n - i0 : chunk, (const W *)(host + buf * kRows));
         }
         return VX3MI_OK;
