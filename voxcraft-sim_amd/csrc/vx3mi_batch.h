@@ -73,10 +73,11 @@ struct RobotTime {
     double scom[3], shist[2][3];
     double recentAngle, closeness;
     int closePairs, angleSamples;
-    // listings beside the steps: per step parity the step whose contacts test every
-    // pair (the lists may miss one), and the step the last listing began
-    int hardStep[2];
-    int listStep;
+    // flat steps whose voxel updates fill the listing grid: per step parity the step
+    // that the lists cannot serve and the step whose updates fill the grid, and whether
+    // the robot ever came to such a step without a grid
+    int hardStep[2], gridStep[2];
+    int jumped;
     int pad;
     int attachUsed;      // pool entries handed out so far (attach)
     int attachOverflow;  // a voxel had more attach candidates than it keeps (kAttachPerVoxel), or the pool ran out

@@ -185,7 +185,7 @@ template <typename T> __device__ __forceinline__ V3<T> cilia_force(const VoxelCi
     return qrot(q, b) * (T)c.coef;
 }
 
-// LISTED: the caller keeps the robots' listing flags (listings beside the steps)
+// LISTED: the caller keeps the robots' listing flags (vx3mi_step.h)
 template <bool LISTED = false, typename T> __device__ __forceinline__ void voxel_update(const Dev<T> &a, int v, int parity) {
     // the loads that need only v (and the link forces, once the link ids are in)
     // are issued before the robot's checks: each check returns early, and a load
@@ -688,16 +688,13 @@ __device__ __forceinline__ int col_list_group(const Dev<T> &a, int s, int v, boo
 }
 
 // The lists of a wave's voxels, kContactLanes lanes each (every lane calls; want:
-// the voxel has one to make), four voxels at a time in kListRounds rounds, or the
-// rounds from r0 on only; returns the count to the voxel's lanes, nc to those with
-// nothing to make.
-constexpr int kListRounds = kListLanes / kContactLanes;
-template <typename T>
-__device__ __forceinline__ int col_list_wave(const Dev<T> &a, int s, int v, bool want, int nc, int r0, int rounds, int *q) {
+// the voxel has one to make), four voxels at a time; returns the count to the
+// voxel's lanes, nc to those with nothing to make.
+template <typename T> __device__ __forceinline__ int col_list_wave(const Dev<T> &a, int s, int v, bool want, int nc, int *q) {
     const int me = threadIdx.x & 63, mine = me / kListLanes;
 #pragma unroll 1
-    for (int k = 0; k < kListRounds; k++) {
-        const bool now = want && mine == k && k >= r0 && k < r0 + rounds;
+    for (int k = 0; k < kListLanes / kContactLanes; k++) {
+        const bool now = want && mine == k;
         if (!__any(now)) continue;
         const int from = k * kListLanes + mine * kContactLanes;
         const int ts = __shfl(s, from), tv = __shfl(v, from);
@@ -709,18 +706,19 @@ __device__ __forceinline__ int col_list_wave(const Dev<T> &a, int s, int v, bool
 }
 
 // where the partners of a contact sum come from: the voxel's candidate list, the
-// grid of the last listing (more candidates than a list holds), or every surface
-// voxel of the robot (a listing beside the steps, when neither is known to hold them all)
+// grid of this step's listing (more candidates than a list holds), or every surface
+// voxel of the robot (lists that may miss one, and no grid to list from)
 enum ColSource { COL_LIST, COL_GRID, COL_ALL };
 
 // the contact force on surface voxel v summed over its kContactLanes lanes (the
 // result is lane 0's), from the state a holds: the lanes take the candidates in
 // turn and add the forces in ascending partner order.  wFirst: this lane's first
-// candidate of a list.  hit: set when a target touches a non-target.
-template <typename T>
+// candidate of a list.  hit: set when a target touches a non-target.  grid(use):
+// calls use(w) for the surface voxels in the grid cells around.
+template <typename T, typename G>
 __device__ __forceinline__ V3<T> col_contact_sum(const Dev<T> &a, const RobotParams &rp, RobotTime *rt, int s, int v, int lane,
                                                  ColSource src, int nc, int wFirst, int matI, int pkv, const T4<T> &qi0,
-                                                 const T4<T> &qi1, const T4<T> &mi0, int &hit) {
+                                                 const T4<T> &qi1, const T4<T> &mi0, int &hit, G &&grid) {
     const int *list = a.clist + (long)s * kMaxCand;
     const VoxelMat &mi = a.vmats[matI];
     const T L = (T)mi.nomSize;
@@ -817,7 +815,7 @@ __device__ __forceinline__ V3<T> col_contact_sum(const Dev<T> &a, const RobotPar
         int prev = -1;
         for (;;) {
             int next = INT_MAX;
-            col_grid_each<false>(a, rp, s, v, [&](int w, const T4<T> &) {
+            grid([&](int w) {
                 if (w > prev && w < next) next = w;
             });
             if (next == INT_MAX) break;
@@ -847,7 +845,7 @@ __device__ __forceinline__ void col_contact(const Dev<T> &a, int s, int parity, 
     const RobotParams &rp = a.rp[r];
     const bool listed = LIST && there && rt->stale[parity] && !rt->diverged;  // the same for the lanes of a voxel
     int nc = ncPre;
-    if constexpr (LIST) nc = col_list_wave(a, s, v, listed, ncPre, 0, kListRounds, q);
+    if constexpr (LIST) nc = col_list_wave(a, s, v, listed, ncPre, q);
     if (!there || !rp.collisions || rt->diverged) return;
     if (!col_active(a, v)) {
         if (lane == 0) a.contactW[v] = T4<T>{0, 0, 0, 0};
@@ -860,7 +858,9 @@ __device__ __forceinline__ void col_contact(const Dev<T> &a, int s, int parity, 
     }
     const V3<T> f = col_contact_sum(a, rp, rt, s, v, lane, nc <= kMaxCand ? COL_LIST : COL_GRID, nc,
                                     listed ? list[lane] : wFirst,  // a listing step has just written the list
-                                    matI, pkv, qi0, qi1, mi0, hit);
+                                    matI, pkv, qi0, qi1, mi0, hit, [&](auto &&use) {
+                                        col_grid_each<false>(a, rp, s, v, [&](int w, const T4<T> &) { use(w); });
+                                    });
     if (lane != 0) return;
     // with signals a non-target voxel touching a target receives a forced 100
     if (hit && !(a.vtarget && a.vtarget[v]) && a.sig && rp.signals) {
@@ -871,13 +871,17 @@ __device__ __forceinline__ void col_contact(const Dev<T> &a, int s, int parity, 
     a.contactW[v] = T4<T>{f.x, f.y, f.z, 0};
 }
 
+// squared distance of two positions of a voxel
+template <typename T> __device__ __forceinline__ T col_moved2(const T4<T> &u, const T4<T> &b) {
+    const T dx = u.x - b.x, dy = u.y - b.y, dz = u.z - b.z;
+    return dx * dx + dy * dy + dz * dz;
+}
+
 // a moved surface voxel marks its robot's lists stale for the next step
 template <typename T> __device__ __forceinline__ void col_track(const Dev<T> &a, int v, const V3<T> &u, RobotTime *rt,
                                                                 const RobotParams &rp, int parity) {
     if (!a.vsurf || a.vsurf[v] < 0) return;
-    const T4<T> b = a.bpos[v];
-    const T dx = u.x - b.x, dy = u.y - b.y, dz = u.z - b.z;
-    if (dx * dx + dy * dy + dz * dz > (T)rp.staleD2) {
+    if (col_moved2(T4<T>{u.x, u.y, u.z, (T)0}, a.bpos[v]) > (T)rp.staleD2) {
         rt->stale[parity ^ 1] = 1;
         a.anyStale[parity ^ 1] = 1;
     }
@@ -896,7 +900,7 @@ template <typename T> __device__ __forceinline__ void col_track(const Dev<T> &a,
 // per-voxel passes (the ranks inside a bucket may differ, which the ascending
 // lists do not see).
 constexpr int kCountPerGroup = 4096;  // four surface voxels per thread of a 1024-thread workgroup
-template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<T> &a, const RobotParams &rp, int s0, int s1, T4<T> *old) {
+template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<T> &a, const RobotParams &rp, int s0, int s1) {
     const double h = rp.listR;
     const int end = s1, nt = blockDim.x;
     for (int i0 = s0 + (int)threadIdx.x; i0 < end; i0 += 4 * nt) {
@@ -921,7 +925,6 @@ template <typename T> __device__ __forceinline__ void col_count_robot(const Dev<
             const int key = (int)(cell_hash(cx, cy, cz) & (unsigned)rp.mask);
             a.scell[s] = int4{cx, cy, cz, key};
             a.srank[s] = atomicAdd(&a.ccnt[rp.toff + key], 1);
-            if (old) old[v[k]] = a.bpos[v[k]];
             a.bpos[v[k]] = q[k];
         }
     }
@@ -955,14 +958,17 @@ template <typename T> __device__ __forceinline__ void col_scatter_robot(const De
     }
 }
 
-// part of the grid of robot r (the calling workgroup's); old: where the positions
-// of the listing before are kept, if anywhere
-template <typename T>
-__device__ __forceinline__ void col_grid_part(const Dev<T> &a, const RobotParams &rp, int r, int part, int *wsum, int &lastPart,
-                                              T4<T> *old = nullptr) {
-    const int parts = (rp.scount + kCountPerGroup - 1) / kCountPerGroup;
+// blockIdx.x: robot r0 + x; blockIdx.y: its part of the count pass
+template <typename T> __global__ __launch_bounds__(1024) void k_col_scan(Dev<T> a, int r0, int parity, int all) {
+    __shared__ int wsum[16];  // wave totals of col_scan
+    __shared__ int lastPart;
+    if (!all && !a.anyStale[parity]) return;
+    const int r = r0 + blockIdx.x;
+    const RobotParams &rp = a.rp[r];
+    if (!a.rt[r].stale[parity] || a.rt[r].diverged || rp.scount == 0) return;
+    const int parts = (rp.scount + kCountPerGroup - 1) / kCountPerGroup, part = blockIdx.y;
     if (part >= parts) return;
-    col_count_robot(a, rp, rp.soff + part * kCountPerGroup, rp.soff + min(rp.scount, (part + 1) * kCountPerGroup), old);
+    col_count_robot(a, rp, rp.soff + part * kCountPerGroup, rp.soff + min(rp.scount, (part + 1) * kCountPerGroup));
     if (parts > 1) {
         // the workgroup that finishes its part last goes on with the whole
         // robot: every workgroup releases its cells, ranks and positions before
@@ -979,17 +985,6 @@ __device__ __forceinline__ void col_grid_part(const Dev<T> &a, const RobotParams
     col_scan<true>(a, r, wsum);
     __syncthreads();
     col_scatter_robot(a, rp);
-}
-
-// blockIdx.x: robot r0 + x; blockIdx.y: its part of the count pass
-template <typename T> __global__ __launch_bounds__(1024) void k_col_scan(Dev<T> a, int r0, int parity, int all) {
-    __shared__ int wsum[16];  // wave totals of col_scan
-    __shared__ int lastPart;
-    if (!all && !a.anyStale[parity]) return;
-    const int r = r0 + blockIdx.x;
-    const RobotParams &rp = a.rp[r];
-    if (!a.rt[r].stale[parity] || a.rt[r].diverged || rp.scount == 0) return;
-    col_grid_part(a, rp, r, blockIdx.y, wsum, lastPart);
 }
 template <typename T> __global__ __launch_bounds__(256) void k_col_contact(Dev<T> a, int s0, int n, int parity) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;  // kContactLanes per surface voxel
@@ -1353,7 +1348,10 @@ template <typename T = int> __global__ __launch_bounds__(1) void k_zero_int(int 
 
 template <typename T> __global__ __launch_bounds__(256) void k_mark_stale(RobotTime *rt, int R, int *anyStale) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < R) rt[r].stale[0] = rt[r].stale[1] = 1;
+    if (r < R) {
+        rt[r].stale[0] = rt[r].stale[1] = 1;
+        rt[r].jumped = 0;
+    }
     if (r == 0 && anyStale) anyStale[0] = anyStale[1] = 1;
 }
 
@@ -1843,7 +1841,6 @@ template <typename T> struct Batch : BatchBase {
             }
         }
         S = (int)surf.size();
-        for (const RobotParams &p : hrp) largeRobot |= p.scount > kListYoungVoxels;
         tableBuckets = buckets;
         HIP_TRY(hipMemcpy(d_rp, hrp.data(), sizeof(RobotParams) * R, hipMemcpyHostToDevice));
         d.contact = nullptr;
@@ -2109,13 +2106,9 @@ template <typename T> struct Batch : BatchBase {
     // scatter; they return at once unless some robot's lists are stale (all:
     // check the robots' own flags only) -- the lists themselves are built by the
     // contact kernels that follow
-    int count_parts(int r0, int nr) const {  // count-pass workgroups of the largest robot
-        int parts = 1;
-        for (int r = r0; r < r0 + nr; r++) parts = std::max(parts, (hrp[r].scount + kCountPerGroup - 1) / kCountPerGroup);
-        return parts;
-    }
     void launch_listing(int r0, int nr, int parity, int all) {
-        const int parts = count_parts(r0, nr);
+        int parts = 1;  // count-pass workgroups of the largest robot
+        for (int r = r0; r < r0 + nr; r++) parts = std::max(parts, (hrp[r].scount + kCountPerGroup - 1) / kCountPerGroup);
         k_col_scan<T><<<dim3(nr, parts), 1024, 0, stream>>>(d, r0, parity, all);
     }
     // the collision phase of one step for surface voxels [s0, s0 + n) (robots
@@ -2143,12 +2136,6 @@ template <typename T> struct Batch : BatchBase {
         if (anySignals) k_signal_deliver<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V);
         if (anyRemoval) k_removal<T><<<(d.nRemCand + 255) / 256, 256, 0, stream>>>(d, parity);
     }
-    ~Batch() override {
-        if (listHardHost) {
-            if (stream) (void)hipStreamSynchronize(stream);  // the last call may still write it
-            (void)hipHostFree(listHardHost);
-        }
-    }
     int kernels_per_flat_step() const {
         return 2 + (anyCollisions ? kCollisionLaunches - 1 : 0) + (anyForceField ? 1 : 0) + (anyRemoval ? 1 : 0) + (anySignals ? 1 : 0) +
                (anyDetach ? 1 : 0) + (anyAttach ? 3 : 0) + (anySample ? 1 : 0);
@@ -2162,53 +2149,37 @@ template <typename T> struct Batch : BatchBase {
 
     Stage<T4<T>> stage;  // reading the state back
 
-    // ---- flat steps with listings beside them (vx3mi_step.h)
-    ListArgs<T> listing = {};
-    int *listHardHost = nullptr;
-    int gridParts = 1;
-    int listLast = 0, listRest = 0;    // steps of the last such call; calls left that list before each step
-    int young = kListYoung;            // steps left that a batch with large robots takes with a listing before each
-    bool largeRobot = false;
+    // ---- flat steps whose updates fill the grid (vx3mi_step.h)
+    ListArgs listing = {};
     bool listBatch() const { return S > 0 && anyCollisions && !anyRemoval && !anyDetach && !anyAttach; }
 
     // with the batch where it steps flat by default, else on first use (0.1 ms)
     int listing_buffers() {
-        if (!listBatch() || listing.bold) return VX3MI_OK;
-        int rc;
-        ListArgs<T> f{};
-        if ((rc = alloc(&f.hard, 2))) return rc;
-        if (!listHardHost) HIP_TRY(hipHostMalloc((void **)&listHardHost, sizeof(int), hipHostMallocDefault));
-        *listHardHost = 0;
-        f.hardHost = listHardHost;
+        if (!listBatch() || listing.node) return VX3MI_OK;
+        ListArgs f{};
         f.nmats = (int)hvmats.size();
-        gridParts = count_parts(0, R);
-        if ((rc = alloc(&f.bold, V))) return rc;
+        int rc;
+        if ((rc = alloc(&f.head, kGridSpread * tableBuckets)) || (rc = alloc(&f.node, V))) return rc;
         listing = f;
+        return listing_serials(0);
+    }
+    // the serial numbers of a run of n steps; they start again, on empty chains, when they run out
+    int listing_serials(unsigned n) {
+        if (listing.serial != 0 && listing.serial < 0xffffffffu - n) return VX3MI_OK;
+        const long n4 = kGridSpread * tableBuckets;
+        k_clear_heads<><<<(int)std::min<long>((n4 + 255) / 256, 4096), 256, 0, stream>>>(listing.head, n4);
+        HIP_TRY(hipGetLastError());
+        listing.serial = 1;
         return VX3MI_OK;
     }
 
-    // Whether a call's flat steps list beside them: enough steps to pay for the
-    // three launches around them, and not a batch whose robots kept crossing the
-    // skin of their lists faster than such a listing follows, so that their steps
-    // tested every pair (a step of that: 0.2 us for each voxel of the robot; more
-    // than 32 voxels' worth a step in the last call): that one lists before each
-    // step for a while.
+    // enough steps to pay for the launches around them
     static constexpr int kListMinSteps = 8;
-    bool list_beside(int nsteps) {
-        if (!listBatch() || nsteps < kListMinSteps) return false;
-        if (listRest > 0) { listRest--; return false; }
-        if (listLast > 0 && *listHardHost / 32 > listLast) {
-            *listHardHost = 0;
-            listRest = 15;
-            return false;
-        }
-        return true;
-    }
 
     void launch_flat_step_listing(int k) {
-        ListArgs<T> f = listing;
+        ListArgs f = listing;
         f.step = k;
-        const int nbg = R * gridParts, nbl = (LP + 255) / 256, nbc = (S * kContactLanes + 255) / 256;
+        const int nbl = (LP + 255) / 256, nbc = (S * kContactLanes + 255) / 256;
         // Force fields beside the contacts: the evaluator's registers leave that launch
         // one wave a SIMD, which a batch that does not fill the device does not notice
         // (us a step with the field beside and after: 1,062 voxels 19.9 and 26.8 in
@@ -2218,9 +2189,9 @@ template <typename T> struct Batch : BatchBase {
         const bool beside = anyForceField && !anyFieldHit && V < 100000;
         if (beside) {
             const int nbf = (V + 255) / 256;
-            k_list_contact_links<T, 1><<<nbg + nbf + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, V, nbf, LP, nbl, S, parity);
+            k_list_contact_links<T, 1><<<nbf + nbl + nbc, 256, 0, stream>>>(d, f, V, nbf, LP, nbl, S, parity);
         } else
-            k_list_contact_links<T, 0><<<nbg + nbl + nbc, 256, 0, stream>>>(d, f, nbg, gridParts, 0, 0, LP, nbl, S, parity);
+            k_list_contact_links<T, 0><<<nbl + nbc, 256, 0, stream>>>(d, f, 0, 0, LP, nbl, S, parity);
         if (anyForceField && !beside) k_force_field<T><<<(V + 255) / 256, 256, 0, stream>>>(d, 0, V, parity);
         k_list_voxels<T><<<(V + 255) / 256, 256, 0, stream>>>(d, f, V, parity);
         if (anySample) k_cycle_sample<T><<<(R + 63) / 64, 64, 0, stream>>>(d, 0, R);
@@ -2229,14 +2200,13 @@ template <typename T> struct Batch : BatchBase {
         launches += 2 + (anyForceField && !beside ? 1 : 0) + (anySample ? 1 : 0) + (anySignals ? 1 : 0);
     }
     int steps_listing(int nsteps) {
-        int rc = listing_buffers();
-        if (rc) return rc;
-        launch_listing(0, R, parity, 0);
-        k_list_begin<T><<<(S * kListLanes + 255) / 256, 256, 0, stream>>>(d, listing, R, S, parity);
+        int rc;
+        if ((rc = listing_buffers()) || (rc = listing_serials((unsigned)nsteps))) return rc;
+        k_list_begin<T><<<(S + 255) / 256, 256, 0, stream>>>(d, listing, R, S, parity);
         for (int k = 0; k < nsteps; k++) launch_flat_step_listing(k);
-        k_list_end<T><<<R, 256, 0, stream>>>(d, listing, nsteps, parity);
-        listLast = nsteps;
-        launches += 3;
+        k_list_end<T><<<(R + 255) / 256, 256, 0, stream>>>(d, R, nsteps, parity);
+        listing.serial += (unsigned)nsteps + 1;
+        launches += 2;
         return VX3MI_OK;
     }
 
@@ -2316,16 +2286,7 @@ template <typename T> struct Batch : BatchBase {
                 parity = (parity + k) & 1;
                 launches++;
             }
-        } else if (listBatch() && largeRobot && young > 0 && nsteps >= kListMinSteps) {
-            const int k = std::min(nsteps, young), rest = nsteps - k;
-            for (int s = 0; s < (rest >= kListMinSteps ? k : nsteps); s++) {
-                launch_flat_step(parity);
-                parity ^= 1;
-                launches += kernels_per_flat_step();
-            }
-            young -= k;
-            if (rest >= kListMinSteps && (rc = steps_listing(rest))) return rc;
-        } else if (list_beside(nsteps)) {
+        } else if (listBatch() && nsteps >= kListMinSteps) {
             if ((rc = steps_listing(nsteps))) return rc;
         } else {
             // 1000-step graphs while at least that many steps remain, then 64-step
@@ -2434,7 +2395,6 @@ template <typename T> struct Batch : BatchBase {
     // the candidate lists of every robot are rebuilt by the next step (after the
     // state was replaced)
     int mark_stale() {
-        young = kListYoung;
         if (!anyCollisions) return VX3MI_OK;
         k_mark_stale<T><<<(R + 255) / 256, 256, 0, stream>>>(d_rt, R, d.anyStale);
         HIP_TRY(hipGetLastError());
