@@ -51,3 +51,25 @@ def test_squeezed_blocks_tiled_equals_plain(precision, dims, squeeze):
     assert np.array_equal(lp[1][~stopped], lt[1][~stopped])  # strains of the running robots
     # a stopped robot's strains are formed again from what its last update left: one more rounding of the rest length
     np.testing.assert_allclose(lt[1][stopped], lp[1][stopped], rtol=4e-7 if precision == vx3mi.FP32 else 0)
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims,E", [((4, 4, 4), 1e9), ((5, 5, 5), 3e8), ((9, 7, 1), 1e9), ((7, 5, 3), 3e8)])
+def test_strains_of_stopped_robots_equal_the_plain_modes(precision, dims, E):
+    """At a timestep too long for their moduli two of four robots pass the divergence
+    strain inside a launch; the tiles form their links' strains again at its end."""
+    n = int(np.prod(dims))
+    base = configs.config0()
+    models = [vx3mi.Model.from_problem(dict(base, dims=dims, cells=(np.arange(n) % 2 + 1).astype(np.int8), phase=np.linspace(0, 1, n),
+                                            enable_collision=1, materials=[dict(configs.SOFT, E=e), dict(configs.SOFT, E=3 * e, cte=0.004)]))
+              for e in (1e6, E, 1e6, 2 * E)]
+    out = []
+    for mode in (vx3mi.MODE_PLAIN, vx3mi.MODE_TILED):
+        b = vx3mi.Batch(models, precision)
+        for k in (1, 30, 40):
+            b.step(k, dt=1e-5, mode=mode)
+        out.append((b.diverged(), *b.link_flags(), b.state()["pos"]))
+        b.close()
+    assert out[0][0].tolist() == [0, 1, 0, 1]
+    for plain, tiled in zip(*out):
+        assert np.array_equal(plain, tiled)
