@@ -1484,6 +1484,7 @@ template <typename T> struct Batch : BatchBase {
         bool ok = false;
         int ntiles = 0;
         int maxLinks = 0;         // of the fullest tile
+        int rounds = 1;           // tiles the device runs one after the other
         int4 *d_tiles = nullptr;  // robot begin, robot count, voxels, links
         int *d_tileRobots = nullptr;
     } plans[2];                   // large and small tile configuration
@@ -2032,6 +2033,7 @@ template <typename T> struct Batch : BatchBase {
             for (int r : b.robots) trobots.push_back(r);
         }
         P.ntiles = (int)tiles.size();
+        P.rounds = (int)((P.ntiles + slots - 1) / slots);
         int rc;
         if ((rc = alloc(&P.d_tiles, tiles.size())) || (rc = alloc(&P.d_tileRobots, trobots.size()))) return rc;
         if (COL && (rc = alloc(&d.tcand, tiles.size() * kMaxCand * C::KV * C::NT))) return rc;
@@ -2048,21 +2050,25 @@ template <typename T> struct Batch : BatchBase {
         if (rc || (rc = plan_tiles_cfg<1, 0>())) return rc;
         tileOK = plans[0].ok || plans[1].ok;
         tileSel = plans[0].ok ? 0 : 1;
-        // The mode of a batch that is not tuned.  A tile's step takes a time that
-        // grows with its links, a flat step one that grows with the whole batch
-        // but starts higher (its launches): microseconds per step, fitted to
-        // batches of 1..400 robots of 3..16 voxels per axis (one robot of 784
-        // voxels, 1,655 links with collisions in FP32: 16.4 tiled, 12.9 flat;
-        // 270 voxels, 550 links: 7.7 and 12.7).  Batches with a robot no tile
-        // holds go flat too: the per-robot kernel is as slow as its largest robot
-        // (200 robots of up to 1,533 links in FP64: 76-119 with 512-256 threads,
-        // flat 69).
+        // The mode of a batch that is not tuned.  A tiled step takes, for each round of
+        // tiles, a time that grows with the fullest tile's links; a flat step one that
+        // grows with the whole batch but starts higher (its launches): microseconds per
+        // step, fitted to batches of 1..4096 robots of 3..12 voxels per axis, up to
+        // 490,000 voxels and five rounds.  Tiled and flat, with collisions in FP32: one
+        // robot of 1,415 links 15.3 and 12.5, four of them 15.2 and 13.3, 64 of them 17.8
+        // and 25.8, one of 1,000 links 10.3 and 12.4; in FP64 one of 457 links 14.3 and
+        // 14.8, 3,072 robots of up to 773 links (five rounds) 85 and 194; without, 3,072
+        // robots 17 and 52, in FP64 (three rounds) 51 and 109.  Batches with a robot no
+        // tile holds go flat too: the per-robot kernel is as slow as its largest robot
+        // (200 robots of up to 1,533 links in FP64: 76-119 with 512-256 threads, flat 43).
         constexpr bool f32 = std::is_same<T, float>::value;
         const bool col = anyCollisions;
         const double tile0 = f32 ? (col ? 4.5 : 3.0) : (col ? 6.4 : 5.5);
-        const double tileLink = f32 ? (col ? 6.6e-3 : 3.3e-3) : (col ? 15.5e-3 : 10.8e-3);
-        const double flat0 = f32 ? (col ? 12.8 : 8.5) : (col ? 16.3 : 14.2), flatVoxel = col ? 1.1e-3 : 8e-5;
-        const bool tiled = tileOK && tile0 + tileLink * plans[tileSel].maxLinks <= flat0 + flatVoxel * V;
+        const double tileLink = f32 ? (col ? 7.0e-3 : 3.3e-3) : (col ? 15.5e-3 : 10.8e-3);
+        const double flat0 = f32 ? (col ? 12.6 : 8.8) : (col ? 15.5 : 14.2);
+        const double flatVoxel = f32 ? (col ? 2.3e-4 : 9.5e-5) : (col ? 3.7e-4 : 2.0e-4);
+        const TilePlan &P = plans[tileSel];
+        const bool tiled = tileOK && (tile0 + tileLink * P.maxLinks) * P.rounds <= flat0 + flatVoxel * V;
         autoMode = tiled ? VX3MI_MODE_TILED : VX3MI_MODE_FLAT;
         return VX3MI_OK;
     }
