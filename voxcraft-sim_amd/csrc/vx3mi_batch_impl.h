@@ -27,6 +27,7 @@
 #include <map>
 #include <cstring>
 #include <new>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -2003,22 +2004,35 @@ template <typename T> struct Batch : BatchBase {
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hrp[x].lcount > hrp[y].lcount; });
         auto pack = [&](long n, bool full) {
             bins.assign((size_t)n, Bin());
+            std::set<std::pair<long, int>> byLoad;  // load, tile (the first of equal loads is found first)
+            for (int b = 0; b < (int)n; b++) byLoad.emplace_hint(byLoad.end(), 0, full ? (int)n - 1 - b : b);
             for (int r : order) {
                 const RobotParams &p = hrp[r];
-                int best = -1;
-                for (int b = 0; b < (int)bins.size(); b++) {
-                    const Bin &x = bins[b];
-                    if (x.l + p.lcount > C::LMAX || x.v + p.vcount > C::VMAX || (int)x.robots.size() >= C::RMAX) continue;
-                    if (best < 0 || (full ? x.l + x.v > bins[best].l + bins[best].v : x.l + x.v < bins[best].l + bins[best].v)) best = b;
-                }
-                if (best < 0) return false;
-                bins[best].l += p.lcount;
-                bins[best].v += p.vcount;
-                bins[best].robots.push_back(r);
+                auto at = [&](const std::pair<long, int> &e) -> Bin & { return bins[full ? n - 1 - e.second : e.second]; };
+                auto room = [&](const std::pair<long, int> &e) {
+                    const Bin &x = at(e);
+                    return x.l + p.lcount <= C::LMAX && x.v + p.vcount <= C::VMAX && (int)x.robots.size() < C::RMAX;
+                };
+                auto it = byLoad.end();
+                if (full) {
+                    const auto back = std::find_if(byLoad.rbegin(), byLoad.rend(), room);
+                    if (back != byLoad.rend()) it = std::prev(back.base());
+                } else
+                    it = std::find_if(byLoad.begin(), byLoad.end(), room);
+                if (it == byLoad.end()) return false;
+                auto node = byLoad.extract(it);
+                Bin &x = at(node.value());
+                x.l += p.lcount;
+                x.v += p.vcount;
+                x.robots.push_back(r);
+                node.value().first = x.l + x.v;
+                byLoad.insert(std::move(node));
             }
             return true;
         };
-        const long least = std::max((totL + C::LMAX - 1) / C::LMAX, (totV + C::VMAX - 1) / C::VMAX);
+        // (robots too: of 80,000 robots of eight voxels a tile holds no more than RMAX,
+        // and each round tried in vain is one more pass over robots and tiles)
+        const long least = std::max<long>({(totL + C::LMAX - 1) / C::LMAX, (totV + C::VMAX - 1) / C::VMAX, (R + C::RMAX - 1l) / C::RMAX});
         for (long rounds = std::max<long>(1, (least + slots - 1) / slots);; rounds++) {
             const long n = std::min<long>(rounds * slots, R);
             if (pack(n, false) || pack(n, true)) break;  // (a tile for each robot always holds them)
