@@ -2176,6 +2176,7 @@ template <typename T> struct Batch : BatchBase {
     // with the batch where it steps flat by default, else on first use (0.1 ms)
     int listing_buffers() {
         if (!listBatch() || listing.node) return VX3MI_OK;
+        OnDevice there(stream);
         ListArgs f{};
         f.nmats = (int)hvmats.size();
         int rc;

@@ -18,6 +18,24 @@
 
 namespace vx3mi {
 
+// the stream's device for as long as this lives: what is made on first use belongs to
+// it, whichever device the calling thread has at the time
+class OnDevice {
+    int before = -1;
+
+public:
+    explicit OnDevice(hipStream_t stream) {
+        int now = -1, its = -1;
+        if (hipGetDevice(&now) == hipSuccess && hipStreamGetDevice(stream, &its) == hipSuccess && now != its && hipSetDevice(its) == hipSuccess)
+            before = now;
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
+
 template <typename W> struct StageRows {  // arrays of n[k] rows
     const W *src[4];
     int n[4];
@@ -39,7 +57,9 @@ template <typename W> class Stage {
 
     // room for the rows of a read, one buffer or two, kept for the next (pinning
     // 1 MB takes 0.13 ms: a small batch holds what it needs)
-    int ready(int need, bool chunks) {
+    int ready(hipStream_t stream, int need, bool chunks) {
+        if (need <= rowsHeld && !(chunks && !done[1])) return VX3MI_OK;
+        OnDevice there(stream);
         for (hipEvent_t &e : done)
             if (chunks && !e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         if (need <= rowsHeld) return VX3MI_OK;
@@ -74,7 +94,7 @@ public:
         }
         const int chunk = kRows / K;
         const bool chunks = n > chunk;
-        int rc = ready(chunks ? 2 * kRows : K * n, chunks);
+        int rc = ready(stream, chunks ? 2 * kRows : K * n, chunks);
         if (rc) return rc;
         auto send = [&](int i0, int buf) -> int {
             const int m = n - i0 < chunk ? n - i0 : chunk;
@@ -83,18 +103,19 @@ public:
             if (chunks) HIP_TRY(hipEventRecord(done[buf], stream));
             return VX3MI_OK;
         };
-        if ((rc = send(0, 0))) return rc;
-        for (int i0 = 0, buf = 0; i0 < n; i0 += chunk, buf ^= 1) {
-            // (a failure leaves the other buffer's chunk in flight: the stream is waited for)
-            if (i0 + chunk < n && (rc = send(i0 + chunk, buf ^ 1))) {
-                (void)hipStreamSynchronize(stream);
-                return rc;
+        // (a failure may leave chunks in flight: the stream is waited for)
+        auto all = [&]() -> int {
+            int rc = send(0, 0);
+            for (int i0 = 0, buf = 0; rc == VX3MI_OK && i0 < n; i0 += chunk, buf ^= 1) {
+                if (i0 + chunk < n && (rc = send(i0 + chunk, buf ^ 1))) break;
+                if (chunks) HIP_TRY(hipEventSynchronize(done[buf]));
+                else HIP_TRY(hipStreamSynchronize(stream));
+                unpack(i0, n - i0 < chunk ? n - i0 : chunk, (const W *)(host + buf * kRows));
             }
-            if (chunks) HIP_TRY(hipEventSynchronize(done[buf]));
-            else HIP_TRY(hipStreamSynchronize(stream));
-            unpack(i0, n - i0 < chunk ? n - i0 : chunk, (const W *)(host + buf * kRows));
-        }
-        return VX3MI_OK;
+            return rc;
+        };
+        if ((rc = all())) (void)hipStreamSynchronize(stream);
+        return rc;
     }
 };
 
