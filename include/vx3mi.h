@@ -39,7 +39,7 @@ extern "C" {
 #define VX3MI_MODE_PLAIN 1       /* one robot per launch sequence (reference-style) */
 #define VX3MI_MODE_FLAT 2        /* one link launch + one voxel launch per step for the whole batch */
 #define VX3MI_MODE_PERSISTENT 3  /* one workgroup per robot, many steps per launch */
-#define VX3MI_MODE_TILED 4       /* robots bin-packed into register/LDS-resident tiles (collisions off) */
+#define VX3MI_MODE_TILED 4       /* robots (or one) bin-packed into register/LDS-resident tiles */
 
 #define VX3MI_MAX_SS_POINTS 32    /* stress-strain data points of a MatModel 3 material */
 #define VX3MI_MAX_CURVE_POINTS 72 /* points of a link's combined stress-strain curve */

@@ -33,7 +33,7 @@ struct DiffBase {
     std::vector<void *> allocs;
     std::vector<RobotParams> hrp;
     std::vector<int> hlat;
-    std::vector<double> hphase0, hE0, hphase, hE;
+    std::vector<double> hphase0, hE0;
     virtual ~DiffBase() {
         for (hipEvent_t e : segEv) (void)hipEventDestroy(e);
         for (void *p : allocs) (void)hipFree(p);

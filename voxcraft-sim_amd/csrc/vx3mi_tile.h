@@ -72,7 +72,6 @@ template <int RMAX, int COL> struct TileRobots {
     double tempAmp[RMAX], tempPeriod[RMAX];  // actuation of each robot (FP32: 1 / period)
     int tempFlags[RMAX];                     // varyTemp | enableExpansion << 1
     int col[RMAX];                           // the robot has collisions (surface voxels in the lists)
-    int spre[RMAX + 1];                      // prefix of the robots' surface voxel counts (collision tiles)
     // collision tiles: the robot lists its candidates at the start of the next
     // step (set by the tracking of the voxel phase), its stale distance, a link
     // of this step passed the divergence strain (merged into diverged once the
@@ -101,13 +100,13 @@ __device__ __forceinline__ int tile_slot(const int *pre, int n, int x) {
 
 // LDSMAT: the batch has at most kTileMatCache voxel and link materials, which
 // are read from LDS in the step loop instead of global memory
-// COL: collision tiles.  Each step, robots whose candidate lists are stale
-// list them first (the tile publishes its poses to global memory and runs the
-// listing passes of the flat path, then packs each voxel's list for the tile);
-// each thread computes the contact forces of its voxels after its links, from
-// the poses and momenta entering the step (LDS) and the packed lists, summed in
-// list order as in k_col_contact.  Tracking and the stale flags stay in LDS
-// during a launch.
+// COL: collision tiles.  Each step, robots whose candidate lists are stale list
+// them first: sixteen lanes to a voxel test its robot's pairs outright, from the
+// poses in LDS, and write its list and the packed words the tile reads.  After the
+// links the lanes of a wave test their voxels' candidates, and what may be in
+// contact is dealt out over the wave for the exact test and the force, from the
+// poses and momenta entering the step (LDS), summed in list order as in
+// k_col_contact.  The stale flags stay in LDS during a launch.
 template <typename T, int SMALL, int LDSMAT, int COL>
 __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL, COL>::C::MINW)) void k_tile(
     Dev<T> a, const int4 *tiles, const int *tileRobots, int nsteps, int parity0, int nLinkMats, int nVoxMats) {
@@ -156,7 +155,6 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
         tr.tempPeriod[tid] = std::is_same<T, float>::value ? p.tempInvPeriod : p.tempPeriod;
         tr.tempFlags[tid] = (p.varyTemp ? 1 : 0) | (p.enableExpansion ? 2 : 0);
         tr.col[tid] = COL && p.collisions && p.scount > 0;
-        tr.spre[tid + 1] = COL ? p.scount : 0;
         if constexpr (COL) {
             tr.stale[tid] = tr.col[tid] && t.stale[parity0 & 1];
             tr.staleD2[tid] = p.staleD2;
@@ -174,12 +172,10 @@ __global__ __launch_bounds__((TileSel<T, SMALL, COL>::C::NT), (TileSel<T, SMALL,
     if (tid == 0) {
         tr.vpre[0] = 0;
         tr.lpre[0] = 0;
-        tr.spre[0] = 0;
         int any = 0;
         for (int j = 0; j < nr; j++) {
             tr.vpre[j + 1] += tr.vpre[j];
             tr.lpre[j + 1] += tr.lpre[j];
-            tr.spre[j + 1] += tr.spre[j];
             if constexpr (COL) any |= tr.stale[j] && !tr.diverged[j];
         }
         tr.anyStale[parity0 & 1] = any;
