@@ -69,3 +69,25 @@ def test_set_moduli_equal_the_models_own(precision, dims):
         assert np.array_equal(sa[k], sb[k]), k
     np.testing.assert_array_equal(pa, pb)
     np.testing.assert_array_equal(ea, eb)
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("dims,robots", [((4, 3, 3), 1), ((7, 6, 6), 1), ((7, 6, 6), 300), ((10, 9, 9), 2)])
+@pytest.mark.parametrize("every", [0, 9])
+def test_each_sweeps_own_choice_equals_the_given_ones(precision, dims, robots, every):
+    """The forward and the reverse steps are laid out each as costs least (7x6x6 robots
+    in FP32: forward by workgroup, reverse flat); given layouts of the reverse sweep
+    and the default give the same bits, with the whole tape and with recomputation."""
+    models = [vx3mi.Model.from_problem(configs.config3(seed=5, dims=dims))] * robots
+    g = np.random.default_rng(3).normal(size=(robots * models[0].nv, 3))
+    out = []
+    for threads in (0, 512 if precision == vx3mi.FP32 else 256, -1):
+        d = vx3mi.Diff(models, precision, checkpoint_every=every, reverse_threads=threads)
+        d.forward(23)
+        out.append((d.state(), *d.backward(grad_pos=g)))
+        d.close()
+    for s, gp, ge in out[1:]:
+        for k in s:
+            assert np.array_equal(s[k], out[0][0][k]), k
+        np.testing.assert_array_equal(gp, out[0][1])
+        np.testing.assert_array_equal(ge, out[0][2])

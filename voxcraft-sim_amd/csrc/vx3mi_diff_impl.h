@@ -188,7 +188,8 @@ template <typename T> struct DiffBatch : DiffBase {
     std::vector<int2v> hends;
     std::vector<int> haxis;
     std::vector<double> hnom;            // link nominal length
-    bool flatSteps = false;              // steps as launches over the whole batch (else one workgroup per robot)
+    // steps as launches over the whole batch (else one workgroup per robot)
+    bool flatForward = false, flatReverse = false;
 
     int create(vx3mi_model *const *models, int n, const vx3mi_diff_opts &opts) {
         R = n;
@@ -282,19 +283,26 @@ template <typename T> struct DiffBatch : DiffBase {
         // Whether a step runs as one item per thread over the whole batch, two
         // launches a phase pair, or as one workgroup per robot: a launch costs more
         // than a workgroup barrier, a robot's items in turn more than the batch's
-        // side by side.  Microseconds per step, forward and reverse together, as
-        // fitted to 1..1000 robots of 3..16 voxels per axis: FP32, one robot of 141
-        // links 13.5 (robot) and 22 (flat), 675 links 25 and 25, 1,344 links 38 and
-        // 26; 128 robots of up to 3,540 links 126 and 56, of up to 250 links 16 and
-        // 27; 1000 robots of up to 469 links 74 and 59.
+        // side by side, unless these have outgrown the caches.  Each sweep by itself,
+        // microseconds per step as fitted to 1..5000 robots of 3..12 voxels per axis,
+        // up to 400,000 voxels (robot and flat): FP32 forward, one robot of 350 links
+        // 6.6 and 9.4, 877 links 10.5 and 10.2, 3,020 links 29.8 and 10.7, 1,500 robots
+        // of up to 588 links 63 and 86, of 225 links 35 and 23; reverse 9.4 and 11.7,
+        // 15.8 and 12.6, 49.7 and 13.4, 105 and 85, 53 and 27.  FP64 forward, 1,500
+        // robots of up to 588 links 147 and 221, reverse 258 and 207.
         constexpr bool f32 = std::is_same<T, float>::value;
         int maxLinks = 0, dev = 0, cus = 256;
         for (const RobotParams &p : hrp) maxLinks = std::max(maxLinks, p.lcount);
         int mp = 0;
         if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&mp, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && mp > 0)
             cus = mp;
-        const double robot = ((f32 ? 12 : 21) + (f32 ? 0.0185 : 0.062) * maxLinks) * ((R + cus - 1) / cus);
-        flatSteps = robot > (f32 ? 24 : 36) + (f32 ? 0.35e-3 : 0.9e-3) * V;
+        auto robot = [&](double base, double link, double voxel) { return (base + link * maxLinks) * ((R + cus - 1) / cus) + voxel * V; };
+        auto flat = [&](double base, double voxel, double beyond) {
+            const int cached = f32 ? 80000 : 40000;
+            return base + voxel * std::min(V, cached) + beyond * std::max(0, V - cached);
+        };
+        flatForward = f32 ? robot(4.6, 8.3e-3, 0) > flat(10.5, 1.2e-4, 2.9e-4) : robot(7.5, 21.5e-3, 0) > flat(15.2, 2.5e-4, 7e-4);
+        flatReverse = f32 ? robot(7.2, 14e-3, 8e-5) > flat(13, 1.2e-4, 2.6e-4) : robot(9, 46e-3, 1.5e-4) > flat(20, 2.5e-4, 6e-4);
 
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         HIP_TRY(hipStreamCreateWithFlags(&rstream, hipStreamNonBlocking));
@@ -440,7 +448,7 @@ template <typename T> struct DiffBatch : DiffBase {
     // (wide: the workgroup size of the per-robot kernel)
     void run_forward(hipStream_t st, int n0, int nsteps, bool wide, int ckEvery, T4<T> *cV, T4<T> *cL, T4<T> *tV, T4<T> *tL,
                      int tapeStart) {
-        if (!flatSteps) {
+        if (!flatForward) {
             for (int s0 = 0; s0 < nsteps; s0 += chunk) {
                 const int k = std::min(chunk, nsteps - s0);
                 if (wide)
@@ -567,7 +575,7 @@ template <typename T> struct DiffBatch : DiffBase {
         const bool recompute = !(tapeValid && nseg == 1);
         // flat: every robot's reverse step at once over the whole device (a robot
         // larger than the others no longer sets the pace of the sweep)
-        const bool flat = optsIn.reverse_threads < 0 || (optsIn.reverse_threads == 0 && flatSteps);
+        const bool flat = optsIn.reverse_threads < 0 || (optsIn.reverse_threads == 0 && flatReverse);
         const bool wide = flat || (optsIn.reverse_threads == DiffThreads<T>::REV_WIDE &&
                                    DiffThreads<T>::REV_WIDE != DiffThreads<T>::REV);
         hipStream_t rs = rstream;
