@@ -272,7 +272,7 @@ __device__ __forceinline__ void step_contact(const Dev<T> &a, const ListArgs &f,
     const int v = a.surf[sv];
     const int r = a.vrob[v], pk = a.lat[v], mat = a.vmat[v];
     const T4<T> q0 = a.pq0[v];
-    const int4 cell = f.node[v];  // (with the rest, where a listing does not wait for it)
+    int4 cell = {0, 0, 0, 0};  // of the grid, in a step that lists
     const float temp = (float)a.pq1[v].w;
     RobotTime *rt = a.rt + r;
     const RobotParams &rp = a.rp[r];
@@ -282,6 +282,7 @@ __device__ __forceinline__ void step_contact(const Dev<T> &a, const ListArgs &f,
     const bool hard = live && rt->hardStep[parity] == f.step;
     const bool lists = hard && rt->gridStep[parity ^ 1] == f.step - 1;
     if (__any(lists)) {
+        cell = f.node[v];
         nc = step_list_wave(a, f, sv, v, lists, nc, q0, cell, pk, mat, rp, room);
         if (lists)
 #pragma unroll
