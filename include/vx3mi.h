@@ -278,9 +278,9 @@ int vx3mi_batch_record_contacts(vx3mi_batch *b, int cap);
 int vx3mi_batch_record_contacts_static(vx3mi_batch *b, int cap);
 /* per robot: the steps whose collision phase rebuilt the robot's candidate
  * lists (every surface voxel lists the surface voxels within its largest
- * contact envelope plus a skin of a quarter voxel; they are rebuilt, through a
- * counting-sort grid, once some surface voxel has moved more than half the
- * skin).  out: n ints. */
+ * contact envelope plus a skin of a quarter voxel, 0.15 voxel for robots of at
+ * most 1,280; they are rebuilt, through a grid, once some surface voxel has moved
+ * more than half the skin).  out: n ints. */
 int vx3mi_batch_listings(vx3mi_batch *b, int *out);
 /* The pairs recorded by the last vx3mi_step call for one robot (robot < 0:
  * all, batch voxel indices): voxel index pairs, the smaller first, sorted.
