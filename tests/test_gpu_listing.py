@@ -254,3 +254,36 @@ def test_a_fast_bodys_steps_cost_a_listing_at_the_most(precision):
         b.close()
     assert listed > 40
     assert us[1] < 8 * us[0], us
+
+
+@pytest.mark.parametrize("precision", [vx3mi.FP32, vx3mi.FP64])
+@pytest.mark.parametrize("far", [60, 700, 1000])
+def test_contacts_between_distant_lattice_sites_equal_the_plain_mode(precision, far):
+    """Two blocks of one robot, far apart in the lattice and put side by side at
+    distances around the contact envelope: their FP32 positions are kept relative to
+    their sites, hundreds of lattice lengths away, where rounding is a fair part of
+    what the first test of a candidate rounds its radius up by."""
+    dims = (far + 3, 3, 3)
+    cells = np.zeros(dims[::-1], np.int8)
+    cells[:, :, :3] = cells[:, :, far:] = 1
+    prob = dict(configs.config0(), dims=dims, cells=cells.reshape(-1), phase=np.linspace(0, 1, 54), enable_collision=1, grav_acc=0.0,
+                floor_enabled=0, materials=[dict(configs.SOFT, cte=0.0)])
+    models = [vx3mi.Model.from_problem(prob)] * 24
+    out = []
+    for mode in (vx3mi.MODE_PLAIN, vx3mi.MODE_FLAT):
+        b = vx3mi.Batch(models, precision)
+        for r in range(24):
+            pos = b.state(r)["pos"]
+            other = pos[:, 0] > 0.01 * (far - 0.5)
+            pos[other, 0] -= 0.01 * far
+            pos[other, 1] += 0.01 * (2 + 1.25 * (1 + (r - 12) * 4e-6))  # the envelope is 1.25 voxels
+            b.set_state(r, pos=pos)
+        b.record_contacts()
+        pairs = []
+        for n in (1, 9, 30):
+            b.step(n, mode=mode)
+            pairs.append(b.contact_pairs())
+        out.append(dict(outcome(b), first=pairs[0], then=pairs[1]))
+        b.close()
+    assert 0 < len(out[0]["first"])
+    assert_same(*out)
